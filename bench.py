@@ -357,9 +357,9 @@ def w13_kernel_name(blk) -> str:
     if blk.shared_fused:
         return (f"moe_gemm_runs_kernel<true, false, false, {pk}> (routed and shared w13 + "
                 "SwiGLU)")
-    ntw = 256 if blk.bm == 256 else 512
-    return (f"moe_gemm_w512_kernel<{blk.bm}, {ntw}, true, false, true, 0> (routed and shared "
-            f"w13 + SwiGLU)")
+    name = ("moe_gemm_t256_kernel<true, false, true, 0>" if blk.bm == 256
+            else f"moe_gemm_w512_kernel<{blk.bm}, true, false, true, 0>")
+    return f"{name} (routed and shared w13 + SwiGLU)"
 
 
 def hbm_traffic(T: int, timeout_s: float = 240.0) -> dict | None:

@@ -107,6 +107,14 @@ constexpr int kPackStride = kPackG * 512;  // elements between a slot's successi
 __host__ __device__ inline int64_t packed_slot_off(int nk, int s) {
   return ((int64_t)(s / kPackG) * nk * kPackG + s % kPackG) * 512;
 }
+// W row (relative to the tile's first `gate` row, or to n0) and k chunk of packed lane l of
+// load instruction i of wave w: the row and chunk the unpacked loads of that slot fetch.
+GLM52_DEV int w512_row(bool gated, int gu_rel, int w, int i, int l) {
+  const int f = i >> 1;
+  const int base = gated ? (f >= 2 ? gu_rel : 0) + w * 64 + (f & 1) * 32 : w * 128 + f * 32;
+  return base + (i & 1) * 8 + phi32(l >> 2);
+}
+GLM52_DEV int w512_chunk(int l) { return (l & 3) ^ (((l >> 2) >> 2) & 3); }
 
 struct GemmArgs {
   const uint16_t* A;
@@ -193,6 +201,15 @@ int launch_wide(const GemmArgs& a, int capacity, bool gated, bool weighted, hipS
 // The 512-row W tile mapping (moe_gemm_wide.hip): GLM52_EUNSUPPORTED for a block size or
 // shape it has no instance for.
 int launch_wide512(const GemmArgs& a, int capacity, bool gated, bool weighted, hipStream_t st);
+
+// The 256 x 256 tile mapping (moe_gemm_t256.hip; block size 256): GLM52_EUNSUPPORTED for a
+// shape it has no instance for.
+int launch_t256(const GemmArgs& a, int capacity, bool gated, bool weighted, hipStream_t st);
+int launch_t256_plain(const GemmArgs& a, int capacity, bool weighted, hipStream_t st);
+int launch_t256_epi(const GemmArgs& a, int capacity, bool weighted, hipStream_t st);
+
+// The record that glm52_debug_item_trace asked the next tile launches to write, or null.
+unsigned long long* item_trace();
 
 // Packs W for launch_wide512 (GemmArgs::Wp): E experts, n_out outputs (gated: the `gate`
 // rows n and the `up` rows gate_up_offset + n), K = k.  Returns the bytes written, or a

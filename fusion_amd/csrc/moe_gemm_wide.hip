@@ -335,26 +335,8 @@ namespace {
 // contiguous memory, a stage of the tile is four 8 KB runs, and the decode weight stream
 // (one slot per item) reads a slot's stages 8 KB apart.
 
-// W row (relative to the tile's first `gate` row, or to n0) and k chunk of packed lane l of
-// load instruction i of wave w: the row and chunk the unpacked loads of that slot fetch.
-GLM52_DEV int w512_row(bool gated, int gu_rel, int w, int i, int l) {
-  const int f = i >> 1;
-  const int base = gated ? (f >= 2 ? gu_rel : 0) + w * 64 + (f & 1) * 32 : w * 128 + f * 32;
-  return base + (i & 1) * 8 + phi32(l >> 2);
-}
-GLM52_DEV int w512_chunk(int l) { return (l & 3) ^ (((l >> 2) >> 2) & 3); }
-
 // EPI (non-gated): 0 bf16 store; 1 bf16(acc + R); 2 C32 += acc (+ R); 3 C32 = acc (fp32
 // partials); 4 the atomic expert merge, bf16 packed atomic adds into row tok / merge_topk.
-//
-// NTW = 512: the tile above (4 waves along W, each 128 W rows x all MT tokens).
-// NTW = 256 (MT = 256): a 256-token x 256-row tile, the waves 2 x 2 (wave (wn, wm): W rows
-// wn * 128 .. +127 against tokens wm * 128 .. +127).  Its W tile is half of a 512-row tile
-// -- gated: `gate` and `up` rows of 128 consecutive outputs -- which the packed layout
-// keeps as 16 KB of contiguous memory per stage (512-row waves 2s and 2s + 1), so both
-// tile heights read one packed copy.  A stage is 32 KB, so five fit in LDS: four in flight
-// while one is multiplied.  A tile of 256 tokens covers most experts' rows at prefill
-// sizes in one item, so most W tiles are streamed by one workgroup only.
 //
 // Dealing.  Each XCD owns a contiguous share of the items (its routed items, then its
 // share of the extra expert's), so the W tiles and token rows its workgroups share stay in
@@ -375,26 +357,22 @@ __device__ __align__(256) int g_w512_deal[kDealSets * kDealStride];
 // The host side of glm52_debug_item_trace: the record the next launches write, or null.
 std::atomic<unsigned long long*> g_item_trace{nullptr};
 
-template <int MT, int NTW, bool GATED, bool WEIGHTED, bool PACKED, int EPI = 0>
+template <int MT, bool GATED, bool WEIGHTED, bool PACKED, int EPI = 0>
 __global__ __launch_bounds__(256) void moe_gemm_w512_kernel(GemmArgs p) {
   const unsigned long long t_start = p.wg_trace ? __builtin_amdgcn_s_memrealtime() : 0ull;
   int n_run = 0;  // items this workgroup ran (the trace record)
   constexpr int BKS = 32;          // k per stage
-  constexpr int WN = NTW / 128;    // waves along W
-  constexpr int WM = 4 / WN;       // waves along the tokens
-  constexpr int TPW = MT / WM;     // tokens per wave
   constexpr int RPI = 16;          // staged rows per load instruction (64 lanes x 16 B / 64 B)
-  constexpr int TF = TPW / 32;     // token blocks of 32 per wave
-  constexpr int NO = GATED ? NTW / 2 : NTW;
-  constexpr int NO512 = GATED ? 256 : 512;  // outputs of a packed 512-row tile
-  constexpr int SPLIT = 512 / NTW;          // W tiles per packed 512-row tile
+  constexpr int NTW = 512;         // W rows per tile, 128 per wave
+  constexpr int TF = MT / 32;      // token blocks of 32 (every wave multiplies all of them)
+  constexpr int NO = GATED ? 256 : 512;  // outputs per tile
   constexpr int WI = NTW / RPI / 4;  // W load instructions per wave and stage
   constexpr int AI = MT / RPI / 4;   // token-row load instructions per wave and stage
   constexpr int IPS = WI + AI;
   constexpr int SROWS = NTW + MT;
   constexpr int SELEM = SROWS * BKS;  // elements per stage
-  constexpr int NSTAGE = 5 * SELEM * 2 <= 163840 ? 5 : 4;
-  static_assert(WN * WM == 4 && AI >= 1 && TF >= 1 && TF <= 4, "tile");
+  constexpr int NSTAGE = 4;
+  static_assert(NSTAGE * SELEM * 2 <= 163840 && AI >= 1 && TF >= 1 && TF <= 4, "tile");
   static_assert((NSTAGE - 2) * IPS < 64, "vmcnt range");
   __shared__ __attribute__((aligned(1024))) uint16_t ring[NSTAGE * SELEM];
 
@@ -402,13 +380,11 @@ __global__ __launch_bounds__(256) void moe_gemm_w512_kernel(GemmArgs p) {
   const int lane = tid % kWave;
   const int wv = tid / kWave;
   const int wvu = __builtin_amdgcn_readfirstlane(wv);
-  const int wn = wvu % WN, wm = wvu / WN;
   const int l32 = lane % 32, h = lane / 32;
 
   const int ntp = *p.ntp;
   const int num_m = ntp / MT;
   const int num_n = p.n_out / NO;
-  const int num_n512 = p.n_out / NO512;
   const int items = num_m * num_n;
   const int nk = p.K / BKS;
   const int per_xcd = (items + 7) / 8;
@@ -484,18 +460,15 @@ __global__ __launch_bounds__(256) void moe_gemm_w512_kernel(GemmArgs p) {
     }
     ++n_run;
     const int n0 = pid_n * NO;
-    const int P = pid_n / SPLIT, sub = pid_n % SPLIT;  // the packed 512-row tile and half
-    // The item's first stage (its stages run from there, wrapping), in the 512-row tiles of
-    // the expert GEMMs (the 64- and 128-token tiles; o_proj's epilogues keep stage 0).  There most W tiles are streamed by
-    // one item, the workgroups advance in step, and with every item at the same stage the
+    // The item's first stage (its stages run from there, wrapping) in the expert GEMMs
+    // (o_proj's epilogues keep stage 0).  There most W tiles are streamed by one item, the workgroups advance in step, and with every item at the same stage the
     // loads in flight sit a multiple of 2 MB apart; starting each expert's tiles 16 stages
     // apart spreads them over the HBM channels (T = 2048: w13 2275 -> 2164 us, w2 1340 ->
-    // 1315 us).  The 256 x 256 tiles keep stage 0 first: there many row blocks share each
-    // W tile through L2 and the same start ran w13 4058 -> 4127 us at T = 8192.  The start
+    // 1315 us).  The start
     // depends on the expert and the 512-row tile only, so packed and in-place W, one launch
     // or separate ones, and the atomic merge (EPI 4) add an output's stages in one order.
-    const int krot = (NTW == 512 && (EPI == 0 || EPI == 4))
-                         ? (((xs ? 0 : e) * num_n512 + P) * 16) % nk
+    const int krot = (EPI == 0 || EPI == 4)
+                         ? (((xs ? 0 : e) * num_n + pid_n) * 16) % nk
                          : 0;
     // the item's operands: the routed rows through the layout, the extra expert's directly
     const uint16_t* Ab = xs ? p.Ax : p.A;
@@ -530,24 +503,24 @@ __global__ __launch_bounds__(256) void moe_gemm_w512_kernel(GemmArgs p) {
     for (int q = 0; q < MT; q += kWave)
       nv_rows += __popcll(__ballot(q + il < MT && tok_of(q + il) < nvalid));
     nv_rows = __builtin_amdgcn_readfirstlane(nv_rows);
-    const int nvf = __builtin_amdgcn_readfirstlane(max(0, min(TF, (nv_rows - wm * TPW + 31) / 32)));
+    const int nvf = __builtin_amdgcn_readfirstlane(min(TF, (nv_rows + 31) / 32));
 
     // W load instruction i of the wave fills slab rows (wv * WI + i) * 16 .. +15 of the
     // tile: packed, 1 KB of contiguous memory; in place, W rows wrow + phi32(lane / 4), 16
     // bytes at logical chunk dc each (the lane's byte offsets inside W[e], < 2^32)
     const uint16_t* wexp = PACKED ? (xs ? p.Wx : p.Wp) +
-                                        (int64_t)(e * num_n512 + P) * packed_tile_elems(nk)
+                                        (int64_t)(e * num_n + pid_n) * packed_tile_elems(nk)
                                   : p.W + (int64_t)e * p.swe;
     uint32_t wvoff[WI];
 #pragma unroll
     for (int i = 0; i < WI; ++i) {
       if (PACKED) {
-        // load slot sub * 32 / SPLIT + wv * WI + i of the 512-row tile: nk KB per slot
-        wvoff[i] = (uint32_t)(packed_slot_off(nk, sub * (32 / SPLIT) + wv * WI + i) * 2 +
+        // load slot wv * WI + i of the tile: nk KB per slot
+        wvoff[i] = (uint32_t)(packed_slot_off(nk, wv * WI + i) * 2 +
                               il * 16);
       } else {
-        const int slab = sub * (NTW / RPI) + wv * WI + i;  // 1 KB slab of the 512-row tile
-        const int row = P * NO512 + w512_row(GATED, p.gu_off, slab / 8, slab % 8, il);
+        const int slab = wv * WI + i;  // 1 KB slab of the tile
+        const int row = pid_n * NO + w512_row(GATED, p.gu_off, slab / 8, slab % 8, il);
         wvoff[i] = (uint32_t)(((int64_t)row * p.swn + dc * 8) * 2);
       }
     }
@@ -583,23 +556,6 @@ __global__ __launch_bounds__(256) void moe_gemm_w512_kernel(GemmArgs p) {
 
     auto run = [&](auto nv_tag) {
       constexpr int NV = decltype(nv_tag)::value;
-      if constexpr (NV == 0) {
-        // no real token in this wave's rows: it still stages its share of every stage
-#pragma unroll
-        for (int st = 0; st < NSTAGE - 1; ++st)
-#pragma unroll
-          for (int i = 0; i < IPS; ++i) issue_one(i, st);
-        GLM52_WAIT_VMCNT((NSTAGE - 2) * IPS);
-        __syncthreads();
-#pragma unroll 1
-        for (int kt = 0; kt < nk; ++kt) {
-          GLM52_WAIT_VMCNT((NSTAGE - 3) * IPS);
-          __syncthreads();
-#pragma unroll
-          for (int i = 0; i < IPS; ++i) issue_one(i, kt + NSTAGE - 1);
-        }
-        return;
-      } else {
       constexpr int NMF = 8 * NV;           // MFMAs per stage
       constexpr int NRD = 8 + 2 * NV;       // fragment reads per stage
       constexpr int NOPS = NRD + IPS;       // reads and loads spread over the MFMAs
@@ -616,10 +572,10 @@ __global__ __launch_bounds__(256) void moe_gemm_w512_kernel(GemmArgs p) {
       auto read_op = [&](int q, const uint16_t* sb, uint4 (&dw)[2][4], uint4 (&da)[2][NV]) {
         if (q < 8) {
           const int ks = q / 4, f = q % 4;
-          dw[ks][f] = *reinterpret_cast<const uint4*>(sb + (wn * 128 + f * 32) * BKS + (ks ? rd1 : rd0));
+          dw[ks][f] = *reinterpret_cast<const uint4*>(sb + (wvu * 128 + f * 32) * BKS + (ks ? rd1 : rd0));
         } else {
           const int ks = (q - 8) / NV, t = (q - 8) % NV;
-          da[ks][t] = *reinterpret_cast<const uint4*>(sb + (NTW + wm * TPW + t * 32) * BKS + (ks ? rd1 : rd0));
+          da[ks][t] = *reinterpret_cast<const uint4*>(sb + (NTW + t * 32) * BKS + (ks ? rd1 : rd0));
         }
       };
 
@@ -679,15 +635,15 @@ __global__ __launch_bounds__(256) void moe_gemm_w512_kernel(GemmArgs p) {
         asm volatile("" : "+v"(ln));
         const int el32 = ln % 32, eh = ln / 32;
         int* const etok =
-            reinterpret_cast<int*>(ring + ((nk - 1) % NSTAGE) * SELEM) + wvu * 2 * TPW;
-        float* const ewgt = reinterpret_cast<float*>(etok + TPW);
-        static_assert(TPW % 64 == 0 && 4 * 2 * TPW * 4 <= SELEM * 2, "epilogue rows");
+            reinterpret_cast<int*>(ring + ((nk - 1) % NSTAGE) * SELEM) + wvu * 2 * MT;
+        float* const ewgt = reinterpret_cast<float*>(etok + MT);
+        static_assert(MT % 64 == 0 && 4 * 2 * MT * 4 <= SELEM * 2, "epilogue rows");
         {
-          int qt[TPW / 64];
+          int qt[MT / 64];
 #pragma unroll
-          for (int j = 0; j < TPW / 64; ++j) qt[j] = tok_of(wm * TPW + j * 64 + ln);
+          for (int j = 0; j < MT / 64; ++j) qt[j] = tok_of(j * 64 + ln);
 #pragma unroll
-          for (int j = 0; j < TPW / 64; ++j) {
+          for (int j = 0; j < MT / 64; ++j) {
             etok[j * 64 + ln] = qt[j];
             if (WEIGHTED) ewgt[j * 64 + ln] = (!xs && qt[j] < nvalid) ? p.topw[qt[j]] : 1.f;
           }
@@ -703,7 +659,7 @@ __global__ __launch_bounds__(256) void moe_gemm_w512_kernel(GemmArgs p) {
               float v[16];
 #pragma unroll
               for (int i = 0; i < 16; ++i) v[i] = silu_mul(acc[fp][t][i], acc[fp + 2][t][i]);
-              uint16_t* dst = crow + n0 + wn * 64 + fp * 32 + eh * 16;
+              uint16_t* dst = crow + n0 + wvu * 64 + fp * 32 + eh * 16;
               *reinterpret_cast<uint4*>(dst) = pack8(v);
               *reinterpret_cast<uint4*>(dst + 8) = pack8(v + 8);
             }
@@ -714,7 +670,7 @@ __global__ __launch_bounds__(256) void moe_gemm_w512_kernel(GemmArgs p) {
               float v[16];
 #pragma unroll
               for (int i = 0; i < 16; ++i) v[i] = WEIGHTED ? acc[f][t][i] * wgt : acc[f][t][i];
-              uint16_t* dst = crow + n0 + wn * 128 + f * 32 + eh * 16;
+              uint16_t* dst = crow + n0 + wvu * 128 + f * 32 + eh * 16;
               *reinterpret_cast<uint4*>(dst) = pack8(v);
               *reinterpret_cast<uint4*>(dst + 8) = pack8(v + 8);
             }
@@ -723,7 +679,7 @@ __global__ __launch_bounds__(256) void moe_gemm_w512_kernel(GemmArgs p) {
       } else {
 #pragma unroll
         for (int t = 0; t < NV; ++t) {  // o_proj epilogues and the atomic merge (plain only)
-          const int tok = tok_of(wm * TPW + t * 32 + l32);
+          const int tok = tok_of(t * 32 + l32);
           if (tok >= nvalid) continue;
           uint16_t* crow = EPI >= 2 ? nullptr : p.C + (int64_t)tok * p.scm;
           float wgt = 1.f;
@@ -733,7 +689,7 @@ __global__ __launch_bounds__(256) void moe_gemm_w512_kernel(GemmArgs p) {
             float v[16];
 #pragma unroll
             for (int i = 0; i < 16; ++i) v[i] = WEIGHTED ? acc[f][t][i] * wgt : acc[f][t][i];
-            const int col = n0 + wn * 128 + f * 32 + h * 16;
+            const int col = n0 + wvu * 128 + f * 32 + h * 16;
             if (EPI == 1 || (EPI == 2 && p.R)) {  // + the residual row, in fp32 (epilogue 3: none)
               const uint16_t* rr = p.R + (int64_t)tok * p.srm + col;
               float rf[16];
@@ -770,7 +726,6 @@ __global__ __launch_bounds__(256) void moe_gemm_w512_kernel(GemmArgs p) {
           }
         }
       }
-      }
     };
     // the next item's index, fetched while this one runs.  The token-row offsets are
     // complete first: a load the compiler still counts as pending where the branch joins
@@ -787,7 +742,6 @@ __global__ __launch_bounds__(256) void moe_gemm_w512_kernel(GemmArgs p) {
                                        __HIP_MEMORY_SCOPE_AGENT);
     }
     switch (nvf) {
-      case 0: run(std::integral_constant<int, 0>{}); break;
       case 1: run(std::integral_constant<int, 1>{}); break;
       case 2: run(std::integral_constant<int, (TF >= 2 ? 2 : 1)>{}); break;
       case 3: run(std::integral_constant<int, (TF >= 3 ? 3 : 1)>{}); break;
@@ -814,13 +768,13 @@ __global__ __launch_bounds__(256) void moe_gemm_w512_kernel(GemmArgs p) {
   }
 }
 
-template <int MT, int NTW, bool GATED, bool WEIGHTED>
+template <int MT, bool GATED, bool WEIGHTED>
 int launch_w512(const GemmArgs& a_in, int capacity, hipStream_t st) {
-  constexpr int NO = GATED ? NTW / 2 : NTW;
+  constexpr int NO = GATED ? 256 : 512;
   static std::atomic<unsigned> next_set{0};
   GemmArgs a = a_in;
   a.deal_set = (int)(next_set.fetch_add(1, std::memory_order_relaxed) % kDealSets);
-  a.wg_trace = g_item_trace.load(std::memory_order_relaxed);
+  a.wg_trace = item_trace();
   if ((a.n_out % (GATED ? 256 : 512)) || (a.K % 64)) return GLM52_EUNSUPPORTED;
   const int x_blocks = (a.Wp && a.Wx && a.x_rows > 0) ? (a.x_rows + MT - 1) / MT : 0;
   const int items_max = (capacity / MT + x_blocks) * (a.n_out / NO);
@@ -829,15 +783,15 @@ int launch_w512(const GemmArgs& a_in, int capacity, hipStream_t st) {
   if constexpr (!GATED && !WEIGHTED) {
     if (a.epi != 0 && !a.Wp) return GLM52_EUNSUPPORTED;
     if (a.epi == 1) {
-      moe_gemm_w512_kernel<MT, NTW, false, false, true, 1><<<grid, 256, 0, st>>>(a);
+      moe_gemm_w512_kernel<MT, false, false, true, 1><<<grid, 256, 0, st>>>(a);
       GLM52_RETURN_LAUNCH();
     }
     if (a.epi == 2) {
-      moe_gemm_w512_kernel<MT, NTW, false, false, true, 2><<<grid, 256, 0, st>>>(a);
+      moe_gemm_w512_kernel<MT, false, false, true, 2><<<grid, 256, 0, st>>>(a);
       GLM52_RETURN_LAUNCH();
     }
     if (a.epi == 3) {
-      moe_gemm_w512_kernel<MT, NTW, false, false, true, 3><<<grid, 256, 0, st>>>(a);
+      moe_gemm_w512_kernel<MT, false, false, true, 3><<<grid, 256, 0, st>>>(a);
       GLM52_RETURN_LAUNCH();
     }
   } else {
@@ -846,27 +800,27 @@ int launch_w512(const GemmArgs& a_in, int capacity, hipStream_t st) {
   if (a.merge_topk > 0) {  // the atomic expert merge: weighted w2 only
     if constexpr (!GATED && WEIGHTED) {
       if (a.Wp)
-        moe_gemm_w512_kernel<MT, NTW, false, true, true, 4><<<grid, 256, 0, st>>>(a);
+        moe_gemm_w512_kernel<MT, false, true, true, 4><<<grid, 256, 0, st>>>(a);
       else
-        moe_gemm_w512_kernel<MT, NTW, false, true, false, 4><<<grid, 256, 0, st>>>(a);
+        moe_gemm_w512_kernel<MT, false, true, false, 4><<<grid, 256, 0, st>>>(a);
       GLM52_RETURN_LAUNCH();
     } else {
       return GLM52_EUNSUPPORTED;
     }
   }
   if (a.Wp)
-    moe_gemm_w512_kernel<MT, NTW, GATED, WEIGHTED, true><<<grid, 256, 0, st>>>(a);
+    moe_gemm_w512_kernel<MT, GATED, WEIGHTED, true><<<grid, 256, 0, st>>>(a);
   else
-    moe_gemm_w512_kernel<MT, NTW, GATED, WEIGHTED, false><<<grid, 256, 0, st>>>(a);
+    moe_gemm_w512_kernel<MT, GATED, WEIGHTED, false><<<grid, 256, 0, st>>>(a);
   GLM52_RETURN_LAUNCH();
 }
 
 template <bool GATED, bool WEIGHTED>
 int launch_w512_bm(const GemmArgs& a, int capacity, hipStream_t st) {
   switch (a.BM) {
-    case 64: return launch_w512<64, 512, GATED, WEIGHTED>(a, capacity, st);
-    case 128: return launch_w512<128, 512, GATED, WEIGHTED>(a, capacity, st);
-    case 256: return launch_w512<256, 256, GATED, WEIGHTED>(a, capacity, st);
+    case 64: return launch_w512<64, GATED, WEIGHTED>(a, capacity, st);
+    case 128: return launch_w512<128, GATED, WEIGHTED>(a, capacity, st);
+    case 256: return launch_t256(a, capacity, GATED, WEIGHTED, st);
     default: return GLM52_EUNSUPPORTED;
   }
 }
@@ -920,6 +874,10 @@ int launch_wide512(const GemmArgs& a, int capacity, bool gated, bool weighted, h
   return weighted ? launch_w512_bm<false, true>(a, capacity, st) : launch_w512_bm<false, false>(a, capacity, st);
 }
 
+}  // namespace glm52
+
+namespace glm52 {
+unsigned long long* item_trace() { return g_item_trace.load(std::memory_order_relaxed); }
 }  // namespace glm52
 
 extern "C" int glm52_debug_item_trace(void* buf, int64_t bytes) {

@@ -291,11 +291,11 @@ Split decode_split(int M, int N, int K) {
   return sp;
 }
 
-// Rows per tile of the prefill mapping: the 256 x 256 tile for 256 .. 2048 rows (it stages
-// a fifth fewer bytes through LDS per flop than 128 rows x 512 columns: o_proj at M = 256
-// 188 -> 148 us, at M = 2048 483 -> 458 us), else 128 rows.  At M = 8192 its twice as many
-// column tiles re-read the 268 MB of A twice as often from HBM (1701 -> 2014 us).
-int prefill_bm(int M) { return M >= 256 && M <= 2048 ? 256 : 128; }
+// Rows per tile of the prefill mapping: the 256 x 256 tile from 256 rows (it stages a fifth
+// fewer bytes through LDS per flop than 128 rows x 512 columns: o_proj at M = 256 188 -> 148
+// us, at M = 2048 483 -> 458 us, and at M = 8192, once an XCD's workgroups took 4 row blocks x
+// 8 column tiles at a time, 1642 -> 1352 us), else 128 rows.
+int prefill_bm(int M) { return M >= 256 ? 256 : 128; }
 
 // K slices of the prefill mapping: enough (1 .. 16, powers of two) to give the 256 CUs
 // about one tile each, keeping every slice a multiple of 64 and at least 1024 k.

@@ -1,0 +1,89 @@
+"""The 256 x 256 tile GEMM (block size 256) at the edges of its tiles, against fp32 torch.
+
+Row counts at the edges of a 16-row group, of a wave's share and of a block; the fewest
+stages and an odd number of ring turns; row blocks of one expert past the groups they are
+ordered in and past the 64 expert ids one look-up loads.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from fusion_amd.dispatch import moe_align_block_size
+from fusion_amd.kernels import moe_gateup as KG
+from fusion_amd.kernels import oproj_resadd as KO
+
+pytestmark = pytest.mark.gpu
+
+BF16 = torch.bfloat16
+
+
+def _close(got, want, K):
+    """bf16 rounding of the result (2^-8 of it, both half-ulps), and K fp32 sums of products
+    whose magnitudes are at most 4 here: K * 4 * 2^-22 covers any order of adds."""
+    err = (got.float() - want).abs()
+    tol = want.abs() * 2.0 ** -8 + K * 4 * 2.0 ** -22
+    assert bool((err <= tol).all()), f"max excess {(err - tol).max().item()}"
+
+
+@pytest.mark.parametrize("rows,K", [((1, 16, 17, 32), 256), ((33, 64, 65, 96), 256),
+                                    ((127, 128, 129, 192), 768), ((193, 255, 256, 257), 256),
+                                    ((1290, 2, 511, 513), 256), ((33 * 256 + 5, 3, 0, 1), 256)])
+def test_tile256_edges(gpu, rows, K):
+    print(f"tile256 rows={rows} K={K}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(sum(rows) + K)
+    E, N, T = len(rows), 512, sum(rows)
+    ids = torch.cat([torch.full((n,), e, dtype=torch.int32) for e, n in enumerate(rows)])
+    ids = ids[torch.randperm(T, generator=torch.Generator().manual_seed(K))].to(gpu)
+    a = torch.empty(T, K, dtype=BF16, device=gpu).normal_(0, 1, generator=g).clamp_(-2, 2)
+    w = torch.empty(E, N, K, dtype=BF16, device=gpu).normal_(0, 1, generator=g).clamp_(-2, 2)
+    tw = torch.rand(T, generator=g, device=gpu)
+    sti, eids, ntp = moe_align_block_size(ids.view(T, 1), 256, E)
+    cfg = {"BLOCK_M": 256}
+    full = torch.empty(T, N, device=gpu)
+    for e in range(E):
+        m = (ids == e).nonzero().view(-1)
+        full[m] = a[m].float() @ w[e].float().t()
+
+    def out(n):
+        return torch.full((T, n), float("nan"), dtype=BF16, device=gpu)
+
+    y, y_p, yw = out(N), out(N), out(N)
+    wp = KG.pack_w512(w, N, 0, False)
+    KG.moe_gemm(a, 1, w, y, None, sti, eids, ntp, T, N, 0, False, cfg)
+    KG.moe_gemm_packed(a, 1, wp, y_p, None, sti, eids, ntp, T, N, False, cfg)
+    KG.moe_gemm_packed(a, 1, wp, yw, tw, sti, eids, ntp, T, N, False, cfg)
+    act, act_p = out(N // 2), out(N // 2)
+    KG.moe_gemm(a, 1, w, act, None, sti, eids, ntp, T, N // 2, N // 2, True, cfg)
+    KG.moe_gemm_packed(a, 1, KG.pack_w512(w, N // 2, N // 2, True), act_p, None, sti, eids, ntp,
+                       T, N // 2, True, cfg)
+    assert torch.equal(y, y_p) and torch.equal(act, act_p)
+    _close(y, full, K)
+    _close(yw, full * tw[:, None], K)
+    gate, up = full[:, :N // 2], full[:, N // 2:]
+    want = torch.nn.functional.silu(gate) * up
+    # silu's slope is at most 1.1: the sums' errors reach the product through both factors
+    err = (act.float() - want).abs()
+    tol = want.abs() * 2.0 ** -7 + (gate.abs() + 1.1 * up.abs() + 1) * K * 4 * 2.0 ** -22
+    assert bool((err <= tol).all())
+
+
+@pytest.mark.parametrize("M,K,N", [(256, 64, 512), (257, 1024, 1024), (700, 2112, 512),
+                                   (2300, 512, 1536)])
+def test_oproj_tile256_edges(gpu, M, K, N):
+    """o_proj from 256 rows: every epilogue, K slices or none, ragged last blocks, and row
+    blocks past one order group."""
+    print(f"oproj tile256 M={M} K={K} N={N}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(M + K)
+    a = torch.empty(M, K, dtype=BF16, device=gpu).normal_(0, 1, generator=g).clamp_(-2, 2)
+    b = torch.empty(K, N, dtype=BF16, device=gpu).normal_(0, 1, generator=g).clamp_(-2, 2)
+    r = torch.empty(M, N, dtype=BF16, device=gpu).normal_(0, 1, generator=g)
+    want = a.float() @ b.float()
+    for res in (None, r):
+        c = torch.full((M, N), float("nan"), dtype=BF16, device=gpu)
+        KO.gemm_launch(a, b, c, res, {}, res is not None, False)
+        _close(c, want if res is None else want + r.float(), K)
+        acc = torch.ones(M, N, device=gpu)
+        KO.gemm_launch(a, b, acc, res, {}, res is not None, True)
+        _close(acc, 1 + (want if res is None else want + r.float()), K)
