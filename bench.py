@@ -357,8 +357,7 @@ def w13_kernel_name(blk) -> str:
     if blk.shared_fused:
         return (f"moe_gemm_runs_kernel<true, false, false, {pk}> (routed and shared w13 + "
                 "SwiGLU)")
-    name = ("moe_gemm_t256_kernel<true, false, true, 0>" if blk.bm == 256
-            else f"moe_gemm_w512_kernel<{blk.bm}, true, false, true, 0>")
+    name = f"moe_gemm_tile_kernel<{blk.bm}, {256 if blk.bm == 256 else 512}, true, false, true, 0>"
     return f"{name} (routed and shared w13 + SwiGLU)"
 
 

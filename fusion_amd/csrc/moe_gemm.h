@@ -198,23 +198,17 @@ GLM52_DEV void atomic_add_bf16x2(uint16_t* p, float lo, float hi) {
 // returns GLM52_EUNSUPPORTED for a block size or shape it has no instance for.
 int launch_wide(const GemmArgs& a, int capacity, bool gated, bool weighted, hipStream_t st);
 
-// The 512-row W tile mapping (moe_gemm_wide.hip): GLM52_EUNSUPPORTED for a block size or
-// shape it has no instance for.
-int launch_wide512(const GemmArgs& a, int capacity, bool gated, bool weighted, hipStream_t st);
-
-// The 256 x 256 tile mapping (moe_gemm_t256.hip; block size 256): GLM52_EUNSUPPORTED for a
-// shape it has no instance for.
-int launch_t256(const GemmArgs& a, int capacity, bool gated, bool weighted, hipStream_t st);
-int launch_t256_plain(const GemmArgs& a, int capacity, bool weighted, hipStream_t st);
-int launch_t256_epi(const GemmArgs& a, int capacity, bool weighted, hipStream_t st);
+// The grouped GEMM tiles at block sizes 64, 128 and 256 (moe_gemm_tile.h): GLM52_EUNSUPPORTED
+// for a block size or shape they have no instance for.
+int launch_tile(const GemmArgs& a, int capacity, bool gated, bool weighted, hipStream_t st);
 
 // The record that glm52_debug_item_trace asked the next tile launches to write, or null.
 unsigned long long* item_trace();
 
-// Packs W for launch_wide512 (GemmArgs::Wp): E experts, n_out outputs (gated: the `gate`
+// Packs W for launch_tile (GemmArgs::Wp): E experts, n_out outputs (gated: the `gate`
 // rows n and the `up` rows gate_up_offset + n), K = k.  Returns the bytes written, or a
 // negative error for a shape the 512-row mapping has no instance for (out = null: size only).
-int64_t pack_wide512(const uint16_t* w, int64_t swe, int64_t swn, int E, int n_out, int k,
+int64_t pack_w512(const uint16_t* w, int64_t swe, int64_t swn, int E, int n_out, int k,
                      int gate_up_offset, bool gated, uint16_t* out, hipStream_t st,
                      int64_t swk = 1);
 

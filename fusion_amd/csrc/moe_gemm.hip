@@ -404,7 +404,7 @@ extern "C" int glm52_moe_gemm(const void* a, int64_t stride_am, int a_row_div, c
   if (variant == 5 || auto_wide) {
     // the 512-row mapping addresses token rows with 32-bit byte offsets; shapes it has no
     // instance for fall back to the 256-row mapping when the mapping was not forced
-    const int rc = g.a_bytes < 0x7ffffff0 ? launch_wide512(g, capacity, gated != 0, weighted, stream)
+    const int rc = g.a_bytes < 0x7ffffff0 ? launch_tile(g, capacity, gated != 0, weighted, stream)
                                           : GLM52_EUNSUPPORTED;
     if (rc != GLM52_EUNSUPPORTED || variant == 5) return rc;
   }
@@ -439,7 +439,7 @@ extern "C" int glm52_moe_gemm(const void* a, int64_t stride_am, int a_row_div, c
 // memory in exactly the order its loads fill LDS.  Same values, same arithmetic: the
 // packed launch computes the same bits as glm52_moe_gemm on the unpacked weights.
 extern "C" int64_t glm52_packed_w512_bytes(int num_experts, int n_out, int k, int gated) {
-  return pack_wide512(nullptr, 0, 0, num_experts, n_out, k, 0, gated != 0, nullptr, nullptr);
+  return pack_w512(nullptr, 0, 0, num_experts, n_out, k, 0, gated != 0, nullptr, nullptr);
 }
 
 extern "C" int glm52_pack_w512(const void* w, int64_t stride_we, int64_t stride_wn,
@@ -449,7 +449,7 @@ extern "C" int glm52_pack_w512(const void* w, int64_t stride_we, int64_t stride_
       stride_wn < k)
     return GLM52_EINVAL;
   if (gated && gate_up_offset < n_out) return GLM52_EINVAL;
-  const int64_t rc = pack_wide512(static_cast<const uint16_t*>(w), stride_we, stride_wn,
+  const int64_t rc = pack_w512(static_cast<const uint16_t*>(w), stride_we, stride_wn,
                                   num_experts, n_out, k, gate_up_offset, gated != 0,
                                   static_cast<uint16_t*>(packed), stream);
   if (rc == GLM52_EUNSUPPORTED) return GLM52_EUNSUPPORTED;
@@ -494,7 +494,7 @@ extern "C" int glm52_moe_down_merge(const void* a, int64_t stride_am, const void
   }
   if (g.a_bytes >= 0x7ffffff0) return GLM52_EUNSUPPORTED;
   g.Wp = static_cast<const uint16_t*>(w_packed);
-  return launch_wide512(g, capacity, false, true, stream);
+  return launch_tile(g, capacity, false, true, stream);
 }
 
 extern "C" int glm52_moe_gemm_packed(const void* a, int64_t stride_am, int a_row_div,
@@ -525,7 +525,7 @@ extern "C" int glm52_moe_gemm_packed(const void* a, int64_t stride_am, int a_row
   g.Wp = static_cast<const uint16_t*>(w_packed);
   if (block_m == 16)  // the contiguous-run weight stream on the packed load slots
     return launch_runs(g, capacity, gated != 0, topk_weights != nullptr, false, stream);
-  return launch_wide512(g, capacity, gated != 0, topk_weights != nullptr, stream);
+  return launch_tile(g, capacity, gated != 0, topk_weights != nullptr, stream);
 }
 
 // glm52_moe_gemm_packed with the shared expert in the same launch (prefill): an extra
@@ -566,7 +566,7 @@ extern "C" int glm52_moe_gemm_packed_shared(
   g.Wp = static_cast<const uint16_t*>(w_packed);
   if (block_m == 16)  // the contiguous-run weight stream on the packed load slots
     return launch_runs(g, capacity, gated != 0, topk_weights != nullptr, false, stream);
-  return launch_wide512(g, capacity, gated != 0, topk_weights != nullptr, stream);
+  return launch_tile(g, capacity, gated != 0, topk_weights != nullptr, stream);
 }
 
 // The routed grouped GEMM and the shared expert's GEMM in one weight-streaming launch

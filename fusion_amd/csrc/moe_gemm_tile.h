@@ -52,19 +52,14 @@ namespace {  // one copy per source file: each has its own counters
 #define GLM52_INLINE __attribute__((always_inline))
 
 constexpr int kRowGroup = 4;
-constexpr int kT = 256;                    // tokens and W rows per tile
 constexpr int kBK = 32;                    // k per stage
-constexpr int kStages = 5;
-constexpr uint32_t kStageBytes = 2 * kT * kBK * 2;
-constexpr uint32_t kRowsBytes = kT * kBK * 2;  // W's part of a stage; the token rows follow
-constexpr int kWI = 4, kAI = 4;            // load instructions per wave, stage and operand
 constexpr uint32_t kNowhere = 0x90000000u;  // past every descriptor: reads zero
 
 // counters the items are dealt from, a set per launch in turn: XCD x's at 16 x, the exits at
 // 128 (see moe_gemm_wide.hip)
 constexpr int kDealSets = 64;
 constexpr int kDealStride = 256;
-__device__ __align__(256) int g_t256_deal[kDealSets * kDealStride];
+__device__ __align__(256) int g_tile_deal[kDealSets * kDealStride];
 
 // f(integral_constant<int, 0>) .. f(integral_constant<int, N - 1>), unrolled at compile time.
 template <int N, int I = 0, typename F>
@@ -137,30 +132,39 @@ GLM52_DEV void drain_and_meet() {
 
 // EPI (non-gated): 0 bf16 store; 1 bf16(acc + R); 2 C32 += acc (+ R); 3 C32 = acc (fp32
 // partials); 4 the atomic expert merge, bf16 packed atomic adds into row tok / merge_topk.
-template <bool GATED, bool WEIGHTED, bool PACKED, int EPI>
-__global__ __launch_bounds__(256) void moe_gemm_t256_kernel(GemmArgs p) {
+template <int MT, int NT, bool GATED, bool WEIGHTED, bool PACKED, int EPI>
+__global__ __launch_bounds__(256) void moe_gemm_tile_kernel(GemmArgs p) {
+  constexpr int kWaveN = NT / 128, kWaveM = 4 / kWaveN;  // waves along W and along the tokens
+  constexpr uint32_t kRowsBytes = NT * kBK * 2;  // W's part of a stage; the token rows follow
+  constexpr uint32_t kStageBytes = (NT + MT) * kBK * 2;
+  constexpr int kStages = 163840 / kStageBytes;
+  constexpr int kWI = NT / 64;  // W load instructions per wave and stage
+  constexpr int kAI = MT / 64;  // token-row load instructions per wave and stage
+  constexpr int kQ = MT / kWave;
   const unsigned long long t_start = p.wg_trace ? __builtin_amdgcn_s_memrealtime() : 0ull;
   int n_run = 0;  // items this workgroup ran (the trace record)
-  constexpr int NO = GATED ? kT / 2 : kT;   // outputs per tile; a packed tile has twice those
+  constexpr int NO = GATED ? NT / 2 : NT;    // outputs per tile; a packed tile has twice those
   __shared__ __attribute__((aligned(1024))) uint16_t ring[kStages * kStageBytes / 2];
+
+  constexpr int kHalves = 512 / NT;  // tiles per packed 512-row tile
 
   const int tid = threadIdx.x;
   const int lane = tid % kWave;
   const int wv = uniform(tid / kWave);
-  const int wn = wv & 1, wm = wv >> 1;
+  const int wn = wv % kWaveN, wm = wv / kWaveN;
   const int r16 = lane & 15, g4 = lane >> 4;
 
-  const int num_m = *p.ntp / kT;
+  const int num_m = *p.ntp / MT;
   const int num_n = p.n_out / NO;
   const int items = num_m * num_n;
   const int nk = p.K / kBK;
   const int per_xcd = (items + 7) / 8;
   // the extra (shared) expert, packed weights only: its items follow each XCD's routed ones
   const bool has_x = PACKED && EPI == 0 && p.Wx && p.x_rows > 0;
-  const int nbx = has_x ? (p.x_rows + kT - 1) / kT : 0;
+  const int nbx = has_x ? (p.x_rows + MT - 1) / MT : 0;
   const int items_x = nbx * num_n;
   const int per_xcd_x = (items_x + 7) / 8;
-  int* const deal = g_t256_deal + p.deal_set * kDealStride;
+  int* const deal = g_tile_deal + p.deal_set * kDealStride;
   const int wg_xcd = gridDim.x / 8;  // workgroups per XCD (the launcher rounds to 8)
 
   const uint32_t ring_base = lds_addr(ring);
@@ -172,9 +176,10 @@ __global__ __launch_bounds__(256) void moe_gemm_t256_kernel(GemmArgs p) {
   int tried = 1;
   int k = blockIdx.x / 8;    // its next item there
   bool xs = false;           // an item of the extra expert
+  int krot = 0;              // its first stage
   bool w_once = false;       // no other item reads this W tile
   int n0 = 0, nv_rows = 0;   // its first output; its real rows, a prefix of the block
-  int tq[kT / kWave];        // the flat token of row q * 64 + lane
+  int tq[kQ];                // the flat token of row q * 64 + lane
   u32x4_t srd_w, srd_a;
   uint32_t w_bytes = 0;
   uint32_t wvoff[PACKED ? 1 : kWI], avoff[kAI];
@@ -229,23 +234,23 @@ __global__ __launch_bounds__(256) void moe_gemm_t256_kernel(GemmArgs p) {
         const int gs = min(kRowGroup, cnt - g0);
         const int in = local - g0 * num_n;
         pid_n = in / gs;
-        row0 = (mb + g0 + in % gs) * kT;
+        row0 = (mb + g0 + in % gs) * MT;
       } else {
         const int Lx = xcd * per_xcd_x + (k - n_r);
         pid_n = Lx / nbx;
-        row0 = (Lx % nbx) * kT;
+        row0 = (Lx % nbx) * MT;
         e = 0;
         w_once = nbx == 1;
       }
       const int nvalid = xs ? p.x_rows : p.num_valid;
       nv_rows = 0;
 #pragma unroll
-      for (int q = 0; q < kT / kWave; ++q) {
+      for (int q = 0; q < kQ; ++q) {
         const int r = row0 + q * kWave + lane;
         tq[q] = xs ? min(r, p.x_rows) : p.sti[r];
       }
 #pragma unroll
-      for (int q = 0; q < kT / kWave; ++q) nv_rows += __popcll(__ballot(tq[q] < nvalid));
+      for (int q = 0; q < kQ; ++q) nv_rows += __popcll(__ballot(tq[q] < nvalid));
       nv_rows = uniform(nv_rows);
       if (nv_rows == 0) {
         k = fetch_now();
@@ -253,13 +258,23 @@ __global__ __launch_bounds__(256) void moe_gemm_t256_kernel(GemmArgs p) {
       }
       ++n_run;
       n0 = pid_n * NO;
+      const int P = pid_n / kHalves, sub = pid_n % kHalves;
 
+      // The item's first stage (its stages run from there, wrapping) in the expert GEMMs on 64-
+      // and 128-token tiles.  There most W tiles are streamed by one item, the workgroups
+      // advance in step, and with every item at the same stage the loads in flight sit a
+      // multiple of 2 MB apart; starting each expert's packed tiles 16 stages apart spreads
+      // them over the HBM channels (T = 1000 block 3262 -> 3237 us).  256-token tiles keep
+      // stage 0: there the tiles of an expert share its token rows stage by stage (T = 8192,
+      // w13 3857 -> 3973 us with the start).  It depends on the expert and the packed tile
+      // only, so packed and in-place W, one launch or separate ones, and the atomic merge add
+      // an output's products in one order.
+      krot = MT <= 128 && (EPI == 0 || EPI == 4) ? ((e * (num_n / kHalves) + P) * 16) % nk : 0;
       // W: the wave's load instruction i fills slab wv * 4 + i (16 rows) of the stage
-      const int P = pid_n / 2, sub = pid_n % 2;
       if constexpr (PACKED) {
         const int64_t tile = packed_tile_elems(nk);
         w_bytes = (uint32_t)(tile * 2);
-        srd_w = make_srd((xs ? p.Wx : p.Wp) + (int64_t)(e * (num_n / 2) + P) * tile, w_bytes);
+        srd_w = make_srd((xs ? p.Wx : p.Wp) + (int64_t)(e * (num_n / kHalves) + P) * tile, w_bytes);
         wvoff[0] = (uint32_t)(packed_slot_off(nk, sub * 16 + wv * kWI) * 2 + lane * 16);
       } else {
         w_bytes = 0xfffffff0u;
@@ -267,20 +282,20 @@ __global__ __launch_bounds__(256) void moe_gemm_t256_kernel(GemmArgs p) {
 #pragma unroll
         for (int i = 0; i < kWI; ++i) {
           const int slab = sub * 16 + wv * kWI + i;
-          const int row = P * (2 * NO) + w512_row(GATED, p.gu_off, slab / 8, slab % 8, lane);
+          const int row = P * (kHalves * NO) + w512_row(GATED, p.gu_off, slab / 8, slab % 8, lane);
           wvoff[i] = (uint32_t)(((int64_t)row * p.swn + w512_chunk(lane) * 8) * 2);
         }
       }
-      // token rows: instruction i fills rows wv * 64 + i * 16 + lane / 4
+      // token rows: instruction i fills rows wv * MT / 4 + i * 16 + lane / 4
       srd_a = make_srd(xs ? p.Ax : p.A, 0x7ffffff0u);
       int tw = tq[0];
 #pragma unroll
-      for (int q = 1; q < kT / kWave; ++q) tw = wv == q ? tq[q] : tw;
+      for (int q = 1; q < kQ; ++q) tw = wv * (MT / 4) / kWave == q ? tq[q] : tw;
 #pragma unroll
       for (int i = 0; i < kAI; ++i) {
-        const int rl = i * 16 + (lane >> 2);
-        const int t = __shfl(tw, rl);
-        avoff[i] = wv * 64 + rl < nv_rows
+        const int rl = wv * (MT / 4) + i * 16 + (lane >> 2);
+        const int t = __shfl(tw, rl % kWave);
+        avoff[i] = rl < nv_rows
                        ? (uint32_t)((xs ? t : t / p.a_div) * (int)(xs ? p.sax : p.sam) +
                                     w512_chunk(lane) * 8) * 2u
                        : kNowhere;
@@ -297,7 +312,9 @@ __global__ __launch_bounds__(256) void moe_gemm_t256_kernel(GemmArgs p) {
   constexpr int WS = PACKED ? kPackStride * 2 : kBK * 2;  // bytes from a stage of W to the next
   auto w_begin = [&]() GLM52_INLINE {  // packed: one stage; in place: a pair
     srd_w[2] = sw >= nk ? 0u : w_bytes;
-    so_w = (uint32_t)sw * WS;
+    int kw = sw + krot;
+    kw = kw >= nk ? kw - nk : kw;
+    so_w = (uint32_t)kw * WS;
     lw = ring_base + wo + (uint32_t)(wv * kWI * 1024);
     wo = next(wo);
     ++sw;
@@ -309,7 +326,9 @@ __global__ __launch_bounds__(256) void moe_gemm_t256_kernel(GemmArgs p) {
   };
   auto a_begin = [&]() GLM52_INLINE {
     srd_a[2] = sa >= nk ? 0u : 0x7ffffff0u;
-    so_a = (uint32_t)sa * (kBK * 2);
+    int ka = sa + krot;
+    ka = ka >= nk ? ka - nk : ka;
+    so_a = (uint32_t)ka * (kBK * 2);
     la = ring_base + ao + kRowsBytes + (uint32_t)(wv * kAI * 1024);
     ao = next(ao);
     la1 = ring_base + ao + kRowsBytes + (uint32_t)(wv * kAI * 1024);
@@ -318,24 +337,30 @@ __global__ __launch_bounds__(256) void moe_gemm_t256_kernel(GemmArgs p) {
   };
   constexpr int WN = PACKED ? kWI : 2 * kWI, AN = 2 * kAI;  // instructions of w_begin / a_begin
   auto w_one = [&](auto nt, int i) GLM52_INLINE {
-    constexpr bool NT = decltype(nt)::value;
+    constexpr bool STREAM = decltype(nt)::value;
     if constexpr (PACKED)
-      dma16b<NT>(srd_w, wvoff[0] + i * 1024, so_w, lw + i * 1024);
+      dma16b<STREAM>(srd_w, wvoff[0] + i * 1024, so_w, lw + i * 1024);
     else  // the two halves of a line by adjacent instructions
-      dma16b<NT>(srd_w, wvoff[i / 2], so_w + (i % 2) * (kBK * 2),
+      dma16b<STREAM>(srd_w, wvoff[i / 2], so_w + (i % 2) * (kBK * 2),
                  ((i % 2) ? lw1 : lw) + (i / 2) * 1024);
   };
   auto a_one = [&](int i) GLM52_INLINE {
     dma16b<false>(srd_a, avoff[i / 2], so_a + (i % 2) * (kBK * 2),
                   ((i % 2) ? la1 : la) + (i / 2) * 1024);
   };
-  // Loads of stage s: even stages the token rows of s + 4 and s + 5 and (packed) W of s + 5 or
-  // (in place) W of s + 4 and s + 5; odd stages W of s + 5 (packed).  The loads younger than
-  // those of stage s + 1 at the start of stage s: packed, W of s + 2 .. s + 4 and one pair of
-  // token rows; in place, one pair of both.
-  constexpr int kLater = PACKED ? 3 * kWI + AN : WN + AN;
-  // the loads younger than those of stage 0 at the end of the prologue
-  constexpr int kLater0 = PACKED ? 4 * kWI + AN : WN + AN;
+  // Stage s loads into the ring, N = kStages: W of stage s + N (packed), and in the stages of
+  // parity kPA the pair s + N - 1, s + N of the token rows (and of W, in place).  later(odd):
+  // the loads younger than the last of stage s + 1's at the start of an even / odd stage s.
+  constexpr int kPA = kStages % 2 ? 0 : 1;
+  auto later = [](bool odd) constexpr {
+    const int pairs = kPA == 0 ? (kStages - 3) / 2 : odd ? (kStages - 4) / 2 : (kStages - 2) / 2;
+    return PACKED ? (kStages - 2) * kWI + pairs * AN : pairs * (WN + AN);
+  };
+  // the loads younger than stage 0's at the end of the prologue, which issues what the stages
+  // -N .. -1 would
+  constexpr int kLater0 =
+      later(true) + (PACKED ? WN + (kPA == 1 ? AN : 0) : (kPA == 1 ? WN + AN : 0));
+  static_assert(kLater0 < 64 && later(false) < 64, "vmcnt range");
   auto prologue_nt = [&](auto nt) GLM52_INLINE {
     auto w_all = [&]() GLM52_INLINE {
       w_begin();
@@ -347,15 +372,11 @@ __global__ __launch_bounds__(256) void moe_gemm_t256_kernel(GemmArgs p) {
 #pragma unroll
       for (int i = 0; i < AN; ++i) a_one(i);
     };
-    a_all();
-    w_all();
-    if constexpr (PACKED) w_all();
-    a_all();
-    w_all();
-    if constexpr (PACKED) {
-      w_all();
-      w_all();
-    }
+    static_for<kStages>([&](auto v) GLM52_INLINE {  // stage v - N
+      constexpr bool pair = (decltype(v)::value + kStages) % 2 == kPA;
+      if constexpr (pair) a_all();
+      if constexpr (PACKED || pair) w_all();
+    });
   };
   auto prologue = [&]() GLM52_INLINE {
     sw = sa = 0;
@@ -391,7 +412,7 @@ __global__ __launch_bounds__(256) void moe_gemm_t256_kernel(GemmArgs p) {
         const int gr = wm * NV + t;
         int o = nvalid;
 #pragma unroll
-        for (int q = 0; q < kT / kWave; ++q) {
+        for (int q = 0; q < kQ; ++q) {
           const int v = __shfl(tq[q], (gr % 4) * 16 + r16);
           o = gr / 4 == q ? v : o;
         }
@@ -432,11 +453,11 @@ __global__ __launch_bounds__(256) void moe_gemm_t256_kernel(GemmArgs p) {
 
       auto stage = [&](auto par_tag) GLM52_INLINE {
         constexpr int PAR = decltype(par_tag)::value;
-        constexpr int NA = PAR == 0 ? AN : 0;
-        constexpr int NW = PACKED || PAR == 0 ? WN : 0;
+        constexpr int NA = PAR == kPA ? AN : 0;
+        constexpr int NW = PACKED || PAR == kPA ? WN : 0;
         // this wave's reads of the stage are done (its buffer is refilled below) and its
         // loads of the next stage have landed, for every wave
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(kLater) : "memory");
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(later(PAR == 1)) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" : : : "memory");
         rdo = next(rdo);
@@ -576,12 +597,15 @@ __global__ __launch_bounds__(256) void moe_gemm_t256_kernel(GemmArgs p) {
         }
       }
     };
-    const int nvg = (c_nv + 31) / 32;  // 16-token groups per wave
+    const int nvg = (c_nv + 16 * kWaveM - 1) / (16 * kWaveM);  // 16-token groups per wave
     auto pick = [&](auto nt) GLM52_INLINE {
-      if (nvg <= 2) run(std::integral_constant<int, 2>{}, nt);
-      else if (nvg <= 4) run(std::integral_constant<int, 4>{}, nt);
-      else if (nvg <= 6) run(std::integral_constant<int, 6>{}, nt);
-      else run(std::integral_constant<int, 8>{}, nt);
+      constexpr int MAXV = MT / (16 * kWaveM);
+      if (MAXV == 2 || nvg <= 2) run(std::integral_constant<int, 2>{}, nt);
+      else if (MAXV == 4 || nvg <= 4) run(std::integral_constant<int, MAXV < 4 ? 2 : 4>{}, nt);
+      else if constexpr (MAXV == 8) {
+        if (nvg <= 6) run(std::integral_constant<int, 6>{}, nt);
+        else run(std::integral_constant<int, 8>{}, nt);
+      }
     };
     if (w_once) pick(std::true_type{});
     else pick(std::false_type{});
@@ -603,25 +627,58 @@ __global__ __launch_bounds__(256) void moe_gemm_t256_kernel(GemmArgs p) {
   }
 }
 
-template <bool GATED, bool WEIGHTED, bool PACKED, int EPI>
-int launch_t256_as(const GemmArgs& a_in, int capacity, hipStream_t st) {
+template <int MT, int NT, bool GATED, bool WEIGHTED, bool PACKED, int EPI>
+int launch_tile_mt(const GemmArgs& a_in, int capacity, hipStream_t st) {
   static std::atomic<unsigned> next_set{0};
   GemmArgs a = a_in;
   a.deal_set = (int)(next_set.fetch_add(1, std::memory_order_relaxed) % kDealSets);
   a.wg_trace = item_trace();
-  const int x_blocks = PACKED && a.Wx && a.x_rows > 0 ? (a.x_rows + kT - 1) / kT : 0;
-  const int items_max = (capacity / kT + x_blocks) * (a.n_out / (GATED ? kT / 2 : kT));
+  const int x_blocks = PACKED && a.Wx && a.x_rows > 0 ? (a.x_rows + MT - 1) / MT : 0;
+  const int items_max = (capacity / MT + x_blocks) * (a.n_out / (GATED ? NT / 2 : NT));
   int grid = items_max < 256 ? items_max : 256;
   grid = ((grid + 7) / 8) * 8;
-  moe_gemm_t256_kernel<GATED, WEIGHTED, PACKED, EPI><<<grid, 256, 0, st>>>(a);
+  moe_gemm_tile_kernel<MT, NT, GATED, WEIGHTED, PACKED, EPI><<<grid, 256, 0, st>>>(a);
   GLM52_RETURN_LAUNCH();
 }
 
-template <bool GATED, bool WEIGHTED, int EPI>
-int launch_t256_w(const GemmArgs& a, int capacity, hipStream_t st) {
-  return a.Wp ? launch_t256_as<GATED, WEIGHTED, true, EPI>(a, capacity, st)
-              : launch_t256_as<GATED, WEIGHTED, false, EPI>(a, capacity, st);
+// W rows per tile: 512 (four waves along W) for the packed expert GEMMs at 64 and 128 tokens,
+// which are weight streams: the token rows are staged half as often (T = 3000 block 3776 ->
+// 3663 us).  256 elsewhere: in place the smaller stage leaves room for a deeper ring, and
+// o_proj has the more items for its few row blocks (M = 64 85 -> 75 us).
+template <int MT, bool GATED, bool WEIGHTED, bool PACKED, int EPI>
+int launch_tile_as(const GemmArgs& a, int capacity, hipStream_t st) {
+  constexpr int NT = MT <= 128 && PACKED && (EPI == 0 || EPI == 4) ? 512 : 256;
+  return launch_tile_mt<MT, NT, GATED, WEIGHTED, PACKED, EPI>(a, capacity, st);
+}
+
+template <int MT, bool GATED, bool WEIGHTED, int EPI>
+int launch_tile_w(const GemmArgs& a, int capacity, hipStream_t st) {
+  return a.Wp ? launch_tile_as<MT, GATED, WEIGHTED, true, EPI>(a, capacity, st)
+              : launch_tile_as<MT, GATED, WEIGHTED, false, EPI>(a, capacity, st);
 }
 
 }  // namespace
+
+template <int MT>
+int launch_tile_gated(const GemmArgs& a, int capacity, bool weighted, hipStream_t st) {
+  return weighted ? launch_tile_w<MT, true, true, 0>(a, capacity, st)
+                  : launch_tile_w<MT, true, false, 0>(a, capacity, st);
+}
+template <int MT>
+int launch_tile_plain(const GemmArgs& a, int capacity, bool weighted, hipStream_t st) {
+  return weighted ? launch_tile_w<MT, false, true, 0>(a, capacity, st)
+                  : launch_tile_w<MT, false, false, 0>(a, capacity, st);
+}
+// o_proj's epilogues (packed B only) and the atomic expert merge (weighted w2 only)
+template <int MT>
+int launch_tile_epi(const GemmArgs& a, int capacity, bool weighted, hipStream_t st) {
+  if (a.merge_topk > 0) {
+    if (!weighted || a.epi != 0) return GLM52_EUNSUPPORTED;
+    return launch_tile_w<MT, false, true, 4>(a, capacity, st);
+  }
+  if (weighted || !a.Wp) return GLM52_EUNSUPPORTED;
+  if (a.epi == 1) return launch_tile_as<MT, false, false, true, 1>(a, capacity, st);
+  if (a.epi == 2) return launch_tile_as<MT, false, false, true, 2>(a, capacity, st);
+  return launch_tile_as<MT, false, false, true, 3>(a, capacity, st);
+}
 }  // namespace glm52

@@ -295,13 +295,13 @@ Split decode_split(int M, int N, int K) {
 // fewer bytes through LDS per flop than 128 rows x 512 columns: o_proj at M = 256 188 -> 148
 // us, at M = 2048 483 -> 458 us, and at M = 8192, once an XCD's workgroups took 4 row blocks x
 // 8 column tiles at a time, 1642 -> 1352 us), else 128 rows.
-int prefill_bm(int M) { return M >= 256 ? 256 : 128; }
+int prefill_bm(int M) { return M >= 256 ? 256 : M > 64 ? 128 : 64; }
 
 // K slices of the prefill mapping: enough (1 .. 16, powers of two) to give the 256 CUs
 // about one tile each, keeping every slice a multiple of 64 and at least 1024 k.
 int prefill_splits(int M, int N, int K) {
   const int bm = prefill_bm(M);
-  const int64_t items = (int64_t)((M + bm - 1) / bm) * (N / (bm == 256 ? 256 : 512));
+  const int64_t items = (int64_t)((M + bm - 1) / bm) * (N / 256);
   int S = 1;
   while (S < 16 && items * S * 2 <= 256 && K % (64 * S * 2) == 0 && K / (S * 2) >= 1024) S *= 2;
   return S;
@@ -337,7 +337,7 @@ extern "C" int glm52_oproj_splits(int M, int N, int K) {
 }
 
 extern "C" int64_t glm52_oproj_packed_bytes(int K, int N) {
-  return pack_wide512(nullptr, 0, 0, 1, N, K, 0, false, nullptr, nullptr);
+  return pack_w512(nullptr, 0, 0, 1, N, K, 0, false, nullptr, nullptr);
 }
 
 // B [K, N] (strides in elements) packed for the prefill mapping, as W = B^T cut into
@@ -348,7 +348,7 @@ extern "C" int glm52_oproj_pack(const void* b, int64_t stride_bk, int64_t stride
       (K % splits))
     return GLM52_EINVAL;
   const int Ks = K / splits;
-  const int64_t rc = pack_wide512(static_cast<const uint16_t*>(b), (int64_t)Ks * stride_bk,
+  const int64_t rc = pack_w512(static_cast<const uint16_t*>(b), (int64_t)Ks * stride_bk,
                                   stride_bn, splits, N, Ks, 0, false,
                                   static_cast<uint16_t*>(packed), stream, stride_bk);
   if (rc == GLM52_EUNSUPPORTED) return GLM52_EUNSUPPORTED;
@@ -423,13 +423,13 @@ extern "C" int glm52_oproj_gemm(const void* a, int64_t stride_am, const void* b,
     g.R = static_cast<const uint16_t*>(r);
     g.srm = stride_rm;
     g.C32 = epi == 2 ? static_cast<float*>(c) : nullptr;
-    return launch_wide512(g, cap, false, false, stream);
+    return launch_tile(g, cap, false, false, stream);
   }
   // fp32 partials [M S][N], then the fixed-order sum over the slices with the epilogue
   g.epi = 3;
   g.C32 = part;
   g.scm = N;
-  const int rc = launch_wide512(g, cap, false, false, stream);
+  const int rc = launch_tile(g, cap, false, false, stream);
   if (rc != GLM52_OK) return rc;
   const hipError_t rerr = launch_reduce(part, N, (int64_t)S * N, S, M, N, r, stride_rm, c,
                                         stride_cm, epi, stream);

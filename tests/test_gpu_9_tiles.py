@@ -1,4 +1,4 @@
-"""The 256 x 256 tile GEMM (block size 256) at the edges of its tiles, against fp32 torch.
+"""The grouped GEMM tiles (block sizes 64, 128, 256) at their edges, against fp32 torch.
 
 Row counts at the edges of a 16-row group, of a wave's share and of a block; the fewest
 stages and an odd number of ring turns; row blocks of one expert past the groups they are
@@ -27,11 +27,12 @@ def _close(got, want, K):
     assert bool((err <= tol).all()), f"max excess {(err - tol).max().item()}"
 
 
+@pytest.mark.parametrize("bm", [64, 128, 256])
 @pytest.mark.parametrize("rows,K", [((1, 16, 17, 32), 256), ((33, 64, 65, 96), 256),
                                     ((127, 128, 129, 192), 768), ((193, 255, 256, 257), 256),
                                     ((1290, 2, 511, 513), 256), ((33 * 256 + 5, 3, 0, 1), 256)])
-def test_tile256_edges(gpu, rows, K):
-    print(f"tile256 rows={rows} K={K}", flush=True)
+def test_tile_edges(gpu, rows, K, bm):
+    print(f"tile bm={bm} rows={rows} K={K}", flush=True)
     g = torch.Generator(device=gpu).manual_seed(sum(rows) + K)
     E, N, T = len(rows), 512, sum(rows)
     ids = torch.cat([torch.full((n,), e, dtype=torch.int32) for e, n in enumerate(rows)])
@@ -39,8 +40,8 @@ def test_tile256_edges(gpu, rows, K):
     a = torch.empty(T, K, dtype=BF16, device=gpu).normal_(0, 1, generator=g).clamp_(-2, 2)
     w = torch.empty(E, N, K, dtype=BF16, device=gpu).normal_(0, 1, generator=g).clamp_(-2, 2)
     tw = torch.rand(T, generator=g, device=gpu)
-    sti, eids, ntp = moe_align_block_size(ids.view(T, 1), 256, E)
-    cfg = {"BLOCK_M": 256}
+    sti, eids, ntp = moe_align_block_size(ids.view(T, 1), bm, E)
+    cfg = {"BLOCK_M": bm}
     full = torch.empty(T, N, device=gpu)
     for e in range(E):
         m = (ids == e).nonzero().view(-1)
@@ -69,12 +70,13 @@ def test_tile256_edges(gpu, rows, K):
     assert bool((err <= tol).all())
 
 
-@pytest.mark.parametrize("M,K,N", [(256, 64, 512), (257, 1024, 1024), (700, 2112, 512),
+@pytest.mark.parametrize("M,K,N", [(17, 64, 512), (64, 2048, 512), (65, 1024, 1536),
+                                   (200, 4160, 512), (256, 64, 512), (257, 1024, 1024), (700, 2112, 512),
                                    (2300, 512, 1536)])
-def test_oproj_tile256_edges(gpu, M, K, N):
-    """o_proj from 256 rows: every epilogue, K slices or none, ragged last blocks, and row
+def test_oproj_tile_edges(gpu, M, K, N):
+    """o_proj from 17 rows: every epilogue, K slices or none, ragged last blocks, and row
     blocks past one order group."""
-    print(f"oproj tile256 M={M} K={K} N={N}", flush=True)
+    print(f"oproj tile M={M} K={K} N={N}", flush=True)
     g = torch.Generator(device=gpu).manual_seed(M + K)
     a = torch.empty(M, K, dtype=BF16, device=gpu).normal_(0, 1, generator=g).clamp_(-2, 2)
     b = torch.empty(K, N, dtype=BF16, device=gpu).normal_(0, 1, generator=g).clamp_(-2, 2)
