@@ -1,4 +1,5 @@
-// Pieces shared by the grouped expert GEMM kernels (moe_gemm.hip, moe_gemm_wide.hip).
+// Pieces shared by the grouped expert GEMM kernels (moe_gemm.hip, moe_gemm_tile.h,
+// moe_gemm_wide.hip, moe_gemm_runs.hip).
 #pragma once
 
 #include "common.h"
@@ -163,10 +164,10 @@ struct GemmArgs {
   int32_t* r_eids;
   int32_t* r_ntp;
   int r_capacity;
-  // 512-row tile mapping: W packed per (expert, tile, 32-k stage) in the order the tile's
+  // prefill tiles: W packed per (expert, tile, 32-k stage) in the order the tile's
   // loads fill LDS (glm52_pack_w512); null: W is read in place
   const uint16_t* Wp;
-  // 512-row tile mapping, plain and unweighted only: epilogue 0 = bf16(acc); 1 =
+  // prefill tiles, plain and unweighted only: epilogue 0 = bf16(acc); 1 =
   // bf16(acc + R); 2 = C32 += acc (+ R if R); 3 = C32 = acc (fp32 partial sums): the
   // dense GEMM + residual of o_proj
   int epi;
@@ -174,13 +175,13 @@ struct GemmArgs {
   int64_t srm;
   float* C32;
   // > 0: the atomic expert merge (FUSE_MERGE): the bf16 result of flat token f is added
-  // with packed bf16 atomics into row f / merge_topk of C (non-gated only; the 512-row
-  // tile and contiguous-run mappings); 0: the result is stored into row f
+  // with packed bf16 atomics into row f / merge_topk of C (non-gated only; the
+  // prefill tiles and the contiguous-run mapping); 0: the result is stored into row f
   int merge_topk;
-  // 512-row tile mapping: the set of per-XCD item counters this launch deals its items
+  // prefill tiles: the set of per-XCD item counters this launch deals its items
   // from (set by the launcher)
   int deal_set;
-  // 512-row tile mapping: null, or a record of 4 words per workgroup (start and end on the
+  // prefill tiles: null, or a record of 4 words per workgroup (start and end on the
   // 100 MHz wall clock, items run, XCD) written at the workgroup's end (glm52_debug_item_trace)
   unsigned long long* wg_trace;
 };
@@ -207,7 +208,7 @@ unsigned long long* item_trace();
 
 // Packs W for launch_tile (GemmArgs::Wp): E experts, n_out outputs (gated: the `gate`
 // rows n and the `up` rows gate_up_offset + n), K = k.  Returns the bytes written, or a
-// negative error for a shape the 512-row mapping has no instance for (out = null: size only).
+// negative error for a shape the packed layout does not hold (out = null: size only).
 int64_t pack_w512(const uint16_t* w, int64_t swe, int64_t swn, int E, int n_out, int k,
                      int gate_up_offset, bool gated, uint16_t* out, hipStream_t st,
                      int64_t swk = 1);

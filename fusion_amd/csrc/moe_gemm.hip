@@ -372,11 +372,11 @@ int a_bytes(int num_valid, int a_div, int64_t sa, int k) {
 
 // variant: 0 = choose: block_m 16 runs the contiguous-run weight stream (6), and the
 // stream mapping (1) for what it does not cover (k % 512 != 0, output rows not 8-byte
-// aligned); block_m 64, 128 and 256 run the 512-row W tiles (5; 256: 256 x 256 tiles), and
+// aligned); block_m 64, 128 and 256 run the prefill tiles (5), and
 // at 64 and 128 the 256-row wide mapping (3) for what those do not cover (gated n_out %
 // 256 != 0, plain n_out % 512 != 0, token rows past 2^31 bytes); any other block_m (32)
-// runs the tiled mapping (2).  1 = stream, 2 = tiled, 3 = wide (64-k stages), 5 = 512-row W
-// tiles (moe_gemm_wide.hip), 6 = contiguous-run weight stream (moe_gemm_runs.hip; block_m
+// runs the tiled mapping (2).  1 = stream, 2 = tiled, 3 = wide (64-k stages), 5 = prefill
+// tiles (moe_gemm_tile.h), 6 = contiguous-run weight stream (moe_gemm_runs.hip; block_m
 // 16) force one mapping.
 extern "C" int glm52_moe_gemm(const void* a, int64_t stride_am, int a_row_div, const void* w,
                               int64_t stride_we, int64_t stride_wn, int gate_up_offset,
@@ -402,7 +402,7 @@ extern "C" int glm52_moe_gemm(const void* a, int64_t stride_am, int a_row_div, c
   const bool weighted = topk_weights != nullptr;
   const bool auto_wide = variant == 0 && (block_m == 64 || block_m == 128 || block_m == 256);
   if (variant == 5 || auto_wide) {
-    // the 512-row mapping addresses token rows with 32-bit byte offsets; shapes it has no
+    // the tiles address token rows with 32-bit byte offsets; shapes they have no
     // instance for fall back to the 256-row mapping when the mapping was not forced
     const int rc = g.a_bytes < 0x7ffffff0 ? launch_tile(g, capacity, gated != 0, weighted, stream)
                                           : GLM52_EUNSUPPORTED;
@@ -433,9 +433,9 @@ extern "C" int glm52_moe_gemm(const void* a, int64_t stride_am, int a_row_div, c
                   : launch_tiled_bm<false, false>(g, capacity, stream);
 }
 
-// Packed weights for the 512-row tile mapping (prefill, block_m 64 or 128).  The mapping
-// reads every 32-k stage of a 512-row W tile as 512 runs of 64 bytes, one per row, which
-// the HBM serves far below its streaming rate; packed, a stage is 32 KB of contiguous
+// Packed weights for the prefill tiles (block_m 64, 128 or 256).  In place a 512-row W tile
+// is read as 512 runs of 128 bytes, one per row and pair of 32-k stages, which the HBM serves
+// below its streaming rate; packed, a stage is 32 KB of contiguous
 // memory in exactly the order its loads fill LDS.  Same values, same arithmetic: the
 // packed launch computes the same bits as glm52_moe_gemm on the unpacked weights.
 extern "C" int64_t glm52_packed_w512_bytes(int num_experts, int n_out, int k, int gated) {
@@ -460,8 +460,8 @@ extern "C" int glm52_pack_w512(const void* w, int64_t stride_we, int64_t stride_
 // the layout, out[f / top_k, :] += bf16(topk_weights[f] * (a[f] . w[e]^T)), each add a
 // packed bf16 atomic (two outputs a word), so the order of a row's adds -- and with it the
 // rounding -- depends on timing.  out [T, n_out] must be seeded by the caller (zeros, or
-// the residual).  w_packed (glm52_pack_w512 of w, may be null) is read by the 512-row tile
-// mapping.  block_m 16 (contiguous-run mapping) or 64 / 128 (512-row tiles).
+// the residual).  w_packed (glm52_pack_w512 of w, may be null) is read by the prefill
+// tiles.  block_m 16 (contiguous-run mapping) or 64 / 128 / 256 (prefill tiles).
 extern "C" int glm52_moe_down_merge(const void* a, int64_t stride_am, const void* w,
                                     int64_t stride_we, int64_t stride_wn, const void* w_packed,
                                     void* out, int64_t stride_om, const float* topk_weights,

@@ -1,19 +1,21 @@
-// 256-token x 256-row grouped GEMM tiles for prefill (about a hundred rows per expert and up),
-// gfx950: the block size 256 of `glm52_moe_gemm*`, and o_proj's prefill tile.  Semantics are
+// Grouped GEMM tiles for prefill (tens to thousands of rows per expert), gfx950: the block
+// sizes 64, 128 and 256 of `glm52_moe_gemm*`, and o_proj from 17 rows.  Semantics are
 // those of the other mappings: `moe_gateup_kernel` (`glm52/kernels/moe_gateup.py:34-148`) when
 // gated, `moe_down_kernel` with MUL_ROUTED_WEIGHT (`glm52/kernels/moe_down_merge.py:66-169`)
 // when weighted, `oproj_gemm_kernel` (`glm52/kernels/oproj_resadd.py:32-136`) for EPI 1-3.
 //
-// Tile.  A workgroup owns one layout block of 256 tokens and 256 rows of that expert's W
-// (gated: the `gate` and `up` rows of 128 consecutive outputs), half of a packed 512-row tile.
-// Four waves, 2 x 2: wave (wn, wm) holds 128 W rows against half of the block's real 16-token
-// groups (nvg of them each, so a part-filled block costs both token halves the same), in
-// `v_mfma_f32_16x16x32_bf16` blocks with W as the first operand.
+// Tile.  A workgroup owns one layout block of MT tokens and NT rows of that expert's W (gated:
+// the `gate` and `up` rows of NT / 2 consecutive outputs): a whole packed 512-row tile or half
+// of one (the choice is at launch_tile_as).  Four waves: each holds 128 W rows, against all of
+// the block's real 16-token groups (NT 512) or half of them (NT 256: 2 x 2 waves, so a
+// part-filled block costs both token halves the same), in `v_mfma_f32_16x16x32_bf16` blocks
+// with W as the first operand.
 //
-// Pipeline.  K advances in 32-k stages through a ring of five 32 KB LDS buffers filled by
-// direct global -> LDS loads.  While the MFMAs of stage s run on fragments already in
-// registers, the wave reads the fragments of stage s + 1 and issues loads for stages s + 4 and
-// s + 5; the order is pinned.  What the loop may not contain was measured on a bare loop: 64
+// Pipeline.  K advances in 32-k stages through a ring of LDS buffers (as many as 160 KB hold:
+// five at 256 x 256) filled by direct global -> LDS loads.  While the MFMAs of stage s run on
+// fragments already in registers, the wave reads the fragments of stage s + 1 and issues loads
+// for the buffer that stage s left; the order is pinned.  What the loop may not contain was
+// measured on the 256 x 256 tile's bare loop: 64
 // MFMAs, 16 fragment reads, 8 loads and a barrier take 1060 cycles a stage (1024 for the MFMAs
 // alone).  A branch per load (a cache-policy choice, a clamp past the last stage) and LDS
 // addresses formed per read made it 1450, so the cache policy is a template argument, the
@@ -30,7 +32,7 @@
 // token rows and shared tiles that other workgroups of the XCD re-read from L2 (T = 8192 with
 // skewed load: w13 3737 -> 3580 us).
 //
-// Order and dealing.  As the 512-row tiles (moe_gemm_wide.hip): expert-aligned contiguous
+// Order and dealing.  The kernel is persistent, one workgroup per CU.  Expert-aligned contiguous
 // shares per XCD, dealt from per-XCD counters; the row blocks of an expert in groups of
 // kRowGroup, so that the 32 workgroups of an XCD read 4 row blocks and 8 column tiles at a
 // time (12 operand tiles for 32 products; column tile by column tile it was 33: o_proj at
@@ -56,7 +58,7 @@ constexpr int kBK = 32;                    // k per stage
 constexpr uint32_t kNowhere = 0x90000000u;  // past every descriptor: reads zero
 
 // counters the items are dealt from, a set per launch in turn: XCD x's at 16 x, the exits at
-// 128 (see moe_gemm_wide.hip)
+// 128; the last workgroup out clears the set
 constexpr int kDealSets = 64;
 constexpr int kDealStride = 256;
 __device__ __align__(256) int g_tile_deal[kDealSets * kDealStride];
@@ -270,7 +272,7 @@ __global__ __launch_bounds__(256) void moe_gemm_tile_kernel(GemmArgs p) {
       // only, so packed and in-place W, one launch or separate ones, and the atomic merge add
       // an output's products in one order.
       krot = MT <= 128 && (EPI == 0 || EPI == 4) ? ((e * (num_n / kHalves) + P) * 16) % nk : 0;
-      // W: the wave's load instruction i fills slab wv * 4 + i (16 rows) of the stage
+      // W: the wave's load instruction i fills slab wv * kWI + i (16 rows) of the stage
       if constexpr (PACKED) {
         const int64_t tile = packed_tile_elems(nk);
         w_bytes = (uint32_t)(tile * 2);
@@ -314,6 +316,7 @@ __global__ __launch_bounds__(256) void moe_gemm_tile_kernel(GemmArgs p) {
     srd_w[2] = sw >= nk ? 0u : w_bytes;
     int kw = sw + krot;
     kw = kw >= nk ? kw - nk : kw;
+    kw = sw >= nk ? 0 : kw;  // the range check is against bytes - so_w: no wrap past the end
     so_w = (uint32_t)kw * WS;
     lw = ring_base + wo + (uint32_t)(wv * kWI * 1024);
     wo = next(wo);
@@ -328,6 +331,7 @@ __global__ __launch_bounds__(256) void moe_gemm_tile_kernel(GemmArgs p) {
     srd_a[2] = sa >= nk ? 0u : 0x7ffffff0u;
     int ka = sa + krot;
     ka = ka >= nk ? ka - nk : ka;
+    ka = sa >= nk ? 0 : ka;
     so_a = (uint32_t)ka * (kBK * 2);
     la = ring_base + ao + kRowsBytes + (uint32_t)(wv * kAI * 1024);
     ao = next(ao);

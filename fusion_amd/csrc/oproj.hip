@@ -20,7 +20,7 @@
 // a row: lane l adds splits l, l + 64, ... in order, then the 64 lane sums meet in a fixed
 // butterfly.  No atomics: the result does not depend on timing.
 //
-// Prefill: the 512-row tile GEMM of the MoE block (moe_gemm_wide.hip) as a one-expert
+// Prefill: the tile GEMM of the MoE block (moe_gemm_tile.h) as a one-expert
 // grouped GEMM over an identity row layout, on a packed copy of B (made once per weight,
 // glm52_oproj_pack), with epilogue 1 or 2 fused.
 #include "moe_gemm.h"
@@ -294,7 +294,8 @@ Split decode_split(int M, int N, int K) {
 // Rows per tile of the prefill mapping: the 256 x 256 tile from 256 rows (it stages a fifth
 // fewer bytes through LDS per flop than 128 rows x 512 columns: o_proj at M = 256 188 -> 148
 // us, at M = 2048 483 -> 458 us, and at M = 8192, once an XCD's workgroups took 4 row blocks x
-// 8 column tiles at a time, 1642 -> 1352 us), else 128 rows.
+// 8 column tiles at a time, 1642 -> 1352 us), else 128 rows, or 64 where they hold
+// every row (with its 256-row tiles, M = 64: 85 -> 75 us).
 int prefill_bm(int M) { return M >= 256 ? 256 : M > 64 ? 128 : 64; }
 
 // K slices of the prefill mapping: enough (1 .. 16, powers of two) to give the 256 CUs

@@ -14,10 +14,10 @@ Same launchers and chain builders as the reference module:
 A is [M, K] bf16, B is [K, N] bf16 with any strides (the reference passes the nn.Linear
 weight transposed and made contiguous).  Decode (M <= 16, B N-contiguous) streams B
 through a split-K kernel with a fixed-order reduction; every other case runs the MoE
-block's 512-row tile GEMM on a packed copy of B, made on first use and cached on the
+block's prefill tile GEMM on a packed copy of B, made on first use and cached on the
 tensor's address, shape, strides and version counter while that tensor lives (an in-place
 update of B re-packs; a new B at a freed B's address re-packs).
-When M gives too few 512-row tiles to fill the GPU (M up to a few hundred), the K range
+When M gives too few tiles to fill the GPU (M up to a few hundred), the K range
 is cut into slices run as separate experts into fp32 partials, summed in slice order.
 Triton mapping keys in `cfg` (BLOCK_M/N/K, GROUP_M, SPLIT_K, num_warps, num_stages) are
 accepted and ignored, except that SPLIT_K > 1 selects the fp32-accumulator chain in the

@@ -267,7 +267,7 @@ int glm52_moe_gemm_packed_shared(const void* a, int64_t stride_am, int a_row_div
  *   glm52_oproj_pack / glm52_oproj_packed_bytes: B packed once as the 512-row tile
  *     mapping's W = B^T, cut into `splits` K slices (no counterpart in the reference);
  *     glm52_oproj_splits(M, N, K) is the count glm52_oproj_gemm wants for that shape
- *     (more slices when M gives too few 512-row tiles to fill the GPU).
+ *     (more slices when M gives too few tiles to fill the GPU).
  *   glm52_cast_add: o = bf16(c (+ r)), c bf16 or fp32 -- oproj_resadd.epilogue_launch
  *     (glm52/kernels/oproj_resadd.py:181-196). */
 int64_t glm52_oproj_workspace_bytes(int M, int N, int K);
