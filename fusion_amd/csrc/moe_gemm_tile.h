@@ -601,10 +601,25 @@ __global__ __launch_bounds__(256) void moe_gemm_tile_kernel(GemmArgs p) {
         }
       }
     };
+    // An instance per 16-token group count, or per even one: a part-filled block then
+    // multiplies up to 32 token rows of padding more.  The odd counts are kept where the matrix
+    // cores and the power limit weigh most, the 256-token expert GEMMs (T = 8192 block 6148 ->
+    // 6074 us).  With them the 64- and 128-token tiles, which wait for their weights, and
+    // o_proj lose (T = 1333 block 3222 -> 3313 us, o_proj at M = 256 131 -> 167 us).
     const int nvg = (c_nv + 16 * kWaveM - 1) / (16 * kWaveM);  // 16-token groups per wave
     auto pick = [&](auto nt) GLM52_INLINE {
       constexpr int MAXV = MT / (16 * kWaveM);
-      if (MAXV == 2 || nvg <= 2) run(std::integral_constant<int, 2>{}, nt);
+      if constexpr (MT == 256 && EPI == 0) {
+        bool done = false;
+        static_for<MAXV - 2>([&](auto v) GLM52_INLINE {  // the least of 2 .. MAXV that holds nvg
+          constexpr int NV = decltype(v)::value + 2;
+          if (!done && nvg <= NV) {
+            run(std::integral_constant<int, NV>{}, nt);
+            done = true;
+          }
+        });
+        if (!done) run(std::integral_constant<int, MAXV>{}, nt);
+      } else if (MAXV == 2 || nvg <= 2) run(std::integral_constant<int, 2>{}, nt);
       else if (MAXV == 4 || nvg <= 4) run(std::integral_constant<int, MAXV < 4 ? 2 : 4>{}, nt);
       else if constexpr (MAXV == 8) {
         if (nvg <= 6) run(std::integral_constant<int, 6>{}, nt);

@@ -30,7 +30,8 @@ def _close(got, want, K):
 @pytest.mark.parametrize("bm", [64, 128, 256])
 @pytest.mark.parametrize("rows,K", [((1, 16, 17, 32), 256), ((33, 64, 65, 96), 256),
                                     ((127, 128, 129, 192), 768), ((193, 255, 256, 257), 256),
-                                    ((1290, 2, 511, 513), 256), ((33 * 256 + 5, 3, 0, 1), 256)])
+                                    ((1290, 2, 511, 513), 256), ((48, 80, 97, 112), 256),
+                                    ((160, 161, 224, 225), 256), ((33 * 256 + 5, 3, 0, 1), 256)])
 def test_tile_edges(gpu, rows, K, bm):
     print(f"tile bm={bm} rows={rows} K={K}", flush=True)
     g = torch.Generator(device=gpu).manual_seed(sum(rows) + K)
