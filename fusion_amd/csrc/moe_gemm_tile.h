@@ -43,6 +43,7 @@
 #pragma once
 
 #include "moe_gemm.h"
+#include "tile_range.h"
 
 #include <atomic>
 #include <type_traits>
@@ -54,8 +55,7 @@ namespace {  // one copy per source file: each has its own counters
 #define GLM52_INLINE __attribute__((always_inline))
 
 constexpr int kRowGroup = 4;
-constexpr int kBK = 32;                    // k per stage
-constexpr uint32_t kNowhere = 0x90000000u;  // past every descriptor: reads zero
+constexpr int kBK = 32;  // k per stage
 
 // counters the items are dealt from, a set per launch in turn: XCD x's at 16 x, the exits at
 // 128; the last workgroup out clears the set
@@ -279,7 +279,7 @@ __global__ __launch_bounds__(256) void moe_gemm_tile_kernel(GemmArgs p) {
         srd_w = make_srd((xs ? p.Wx : p.Wp) + (int64_t)(e * (num_n / kHalves) + P) * tile, w_bytes);
         wvoff[0] = (uint32_t)(packed_slot_off(nk, sub * 16 + wv * kWI) * 2 + lane * 16);
       } else {
-        w_bytes = 0xfffffff0u;
+        w_bytes = kInPlaceBytes;
         srd_w = make_srd(p.W + (int64_t)e * p.swe, w_bytes);
 #pragma unroll
         for (int i = 0; i < kWI; ++i) {
@@ -289,7 +289,7 @@ __global__ __launch_bounds__(256) void moe_gemm_tile_kernel(GemmArgs p) {
         }
       }
       // token rows: instruction i fills rows wv * MT / 4 + i * 16 + lane / 4
-      srd_a = make_srd(xs ? p.Ax : p.A, 0x7ffffff0u);
+      srd_a = make_srd(xs ? p.Ax : p.A, kTokenBytes);
       int tw = tq[0];
 #pragma unroll
       for (int q = 1; q < kQ; ++q) tw = wv * (MT / 4) / kWave == q ? tq[q] : tw;
@@ -309,15 +309,14 @@ __global__ __launch_bounds__(256) void moe_gemm_tile_kernel(GemmArgs p) {
   // ---- the ring -------------------------------------------------------------------------
   // W: stage sw is next, at ring offset wo; token rows: the pair of stages sa, sa + 1
   int sw = 0, sa = 0;
-  uint32_t wo = 0, ao = 0, so_w = 0, so_a = 0, lw = 0, lw1 = 0, la = 0, la1 = 0;
+  uint32_t wo = 0, ao = 0, so_w = 0, so_w1 = 0, so_a = 0, so_a1 = 0, lw = 0, lw1 = 0, la = 0, la1 = 0;
   auto next = [&](uint32_t o) GLM52_INLINE { return o == (kStages - 1) * kStageBytes ? 0u : o + kStageBytes; };
   constexpr int WS = PACKED ? kPackStride * 2 : kBK * 2;  // bytes from a stage of W to the next
   auto w_begin = [&]() GLM52_INLINE {  // packed: one stage; in place: a pair
-    srd_w[2] = sw >= nk ? 0u : w_bytes;
-    int kw = sw + krot;
-    kw = kw >= nk ? kw - nk : kw;
-    kw = sw >= nk ? 0 : kw;  // the range check is against bytes - so_w: no wrap past the end
-    so_w = (uint32_t)kw * WS;
+    const StageLoad l = stage_load(sw, nk, krot, WS, w_bytes);
+    srd_w[2] = l.bytes;
+    so_w = l.off;
+    so_w1 = l.off1;
     lw = ring_base + wo + (uint32_t)(wv * kWI * 1024);
     wo = next(wo);
     ++sw;
@@ -328,11 +327,10 @@ __global__ __launch_bounds__(256) void moe_gemm_tile_kernel(GemmArgs p) {
     }
   };
   auto a_begin = [&]() GLM52_INLINE {
-    srd_a[2] = sa >= nk ? 0u : 0x7ffffff0u;
-    int ka = sa + krot;
-    ka = ka >= nk ? ka - nk : ka;
-    ka = sa >= nk ? 0 : ka;
-    so_a = (uint32_t)ka * (kBK * 2);
+    const StageLoad l = stage_load(sa, nk, krot, kBK * 2, kTokenBytes);
+    srd_a[2] = l.bytes;
+    so_a = l.off;
+    so_a1 = l.off1;
     la = ring_base + ao + kRowsBytes + (uint32_t)(wv * kAI * 1024);
     ao = next(ao);
     la1 = ring_base + ao + kRowsBytes + (uint32_t)(wv * kAI * 1024);
@@ -345,11 +343,11 @@ __global__ __launch_bounds__(256) void moe_gemm_tile_kernel(GemmArgs p) {
     if constexpr (PACKED)
       dma16b<STREAM>(srd_w, wvoff[0] + i * 1024, so_w, lw + i * 1024);
     else  // the two halves of a line by adjacent instructions
-      dma16b<STREAM>(srd_w, wvoff[i / 2], so_w + (i % 2) * (kBK * 2),
-                 ((i % 2) ? lw1 : lw) + (i / 2) * 1024);
+      dma16b<STREAM>(srd_w, wvoff[i / 2], (i % 2) ? so_w1 : so_w,
+                     ((i % 2) ? lw1 : lw) + (i / 2) * 1024);
   };
   auto a_one = [&](int i) GLM52_INLINE {
-    dma16b<false>(srd_a, avoff[i / 2], so_a + (i % 2) * (kBK * 2),
+    dma16b<false>(srd_a, avoff[i / 2], (i % 2) ? so_a1 : so_a,
                   ((i % 2) ? la1 : la) + (i / 2) * 1024);
   };
   // Stage s loads into the ring, N = kStages: W of stage s + N (packed), and in the stages of
