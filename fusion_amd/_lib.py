@@ -86,6 +86,7 @@ QUERIES: dict[str, tuple[list, type]] = {
     "glm52_oproj_workspace_bytes": ([_I, _I, _I], c_int64),
     "glm52_oproj_packed_bytes": ([_I, _I], c_int64),
     "glm52_oproj_splits": ([_I, _I, _I], c_int),
+    "glm52_debug_item_set": ([], c_int),
 }
 
 ERRORS = {-1: "invalid argument", -2: "unsupported argument combination"}

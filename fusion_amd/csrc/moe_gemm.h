@@ -206,6 +206,9 @@ int launch_tile(const GemmArgs& a, int capacity, bool gated, bool weighted, hipS
 // The record that glm52_debug_item_trace asked the next tile launches to write, or null.
 unsigned long long* item_trace();
 
+// Keeps `set` for glm52_debug_item_set (the calling thread's last tile launch); returns it.
+int note_item_set(int set);
+
 // Packs W for launch_tile (GemmArgs::Wp): E experts, n_out outputs (gated: the `gate`
 // rows n and the `up` rows gate_up_offset + n), K = k.  Returns the bytes written, or a
 // negative error for a shape the packed layout does not hold (out = null: size only).

@@ -49,7 +49,7 @@
 #include <type_traits>
 
 namespace glm52 {
-namespace {  // one copy per source file: each has its own counters
+namespace {  // one copy per source file: each has its own counters and their sequence
 
 // the kernel's lambdas share its state by reference, which stays in registers only inlined
 #define GLM52_INLINE __attribute__((always_inline))
@@ -57,11 +57,29 @@ namespace {  // one copy per source file: each has its own counters
 constexpr int kRowGroup = 4;
 constexpr int kBK = 32;  // k per stage
 
-// counters the items are dealt from, a set per launch in turn: XCD x's at 16 x, the exits at
-// 128; the last workgroup out clears the set
-constexpr int kDealSets = 64;
+// Counters the items are dealt from, a set per launch: XCD x's at 16 x, the exits at 128; the
+// last workgroup out clears the set.  Two launches on one set would each run part of the items,
+// so launches in flight together need sets of their own.  Every instance of the source file
+// draws from the one sequence beside the array: an eager launch takes the next of kDealSets
+// sets, so it shares one only with a launch a whole multiple of kDealSets before it; a captured
+// launch takes the next of another kDealSets and keeps it in the graph, so eager launches never
+// meet it (replays that overlap must be of graphs whose captured launches use different sets).
+constexpr int kDealSets = 1024;
 constexpr int kDealStride = 256;
-__device__ __align__(256) int g_tile_deal[kDealSets * kDealStride];
+__device__ __align__(256) int g_tile_deal[2 * kDealSets * kDealStride];
+std::atomic<unsigned> g_next_eager{0}, g_next_captured{0};
+
+int take_deal_set(hipStream_t st) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
+    (void)hipGetLastError();  // the launch reports its own error
+    cap = hipStreamCaptureStatusNone;
+  }
+  const bool captured = cap != hipStreamCaptureStatusNone;
+  std::atomic<unsigned>& next = captured ? g_next_captured : g_next_eager;
+  const int set = (int)(next.fetch_add(1, std::memory_order_relaxed) % kDealSets);
+  return note_item_set(captured ? kDealSets + set : set);
+}
 
 // f(integral_constant<int, 0>) .. f(integral_constant<int, N - 1>), unrolled at compile time.
 template <int N, int I = 0, typename F>
@@ -646,9 +664,8 @@ __global__ __launch_bounds__(256) void moe_gemm_tile_kernel(GemmArgs p) {
 
 template <int MT, int NT, bool GATED, bool WEIGHTED, bool PACKED, int EPI>
 int launch_tile_mt(const GemmArgs& a_in, int capacity, hipStream_t st) {
-  static std::atomic<unsigned> next_set{0};
   GemmArgs a = a_in;
-  a.deal_set = (int)(next_set.fetch_add(1, std::memory_order_relaxed) % kDealSets);
+  a.deal_set = take_deal_set(st);
   a.wg_trace = item_trace();
   const int x_blocks = PACKED && a.Wx && a.x_rows > 0 ? (a.x_rows + MT - 1) / MT : 0;
   const int items_max = (capacity / MT + x_blocks) * (a.n_out / (GATED ? NT / 2 : NT));

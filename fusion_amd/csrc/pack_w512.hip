@@ -1,5 +1,5 @@
 // The writer of the packed weight layout, which the grouped GEMM tiles (moe_gemm_tile.h) and
-// the decode kernels read, and the tiles' measurement hook.
+// the decode kernels read, and the tiles' debugging hooks.
 #include "moe_gemm.h"
 
 #include <atomic>
@@ -10,6 +10,9 @@ namespace {
 
 // The host side of glm52_debug_item_trace: the record the next launches write, or null.
 std::atomic<unsigned long long*> g_item_trace{nullptr};
+
+// The host side of glm52_debug_item_set.
+thread_local int t_item_set = -1;
 
 // One 16-byte chunk of the packed layout per thread and step: chunk d is lane d % 64 of
 // stage (d / 64) % nk of load slot (d / (64 nk)) % 32 of tile d / (2048 nk), written at
@@ -56,6 +59,7 @@ __global__ __launch_bounds__(256) void pack_w512_kernel(const uint16_t* __restri
 
 namespace glm52 {
 unsigned long long* item_trace() { return g_item_trace.load(std::memory_order_relaxed); }
+int note_item_set(int set) { return t_item_set = set; }
 }  // namespace glm52
 
 extern "C" int glm52_debug_item_trace(void* buf, int64_t bytes) {
@@ -63,6 +67,8 @@ extern "C" int glm52_debug_item_trace(void* buf, int64_t bytes) {
   g_item_trace.store(static_cast<unsigned long long*>(buf), std::memory_order_relaxed);
   return GLM52_OK;
 }
+
+extern "C" int glm52_debug_item_set(void) { return t_item_set; }
 
 namespace glm52 {
 int64_t pack_w512(const uint16_t* w, int64_t swe, int64_t swn, int E, int n_out, int k,

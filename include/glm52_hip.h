@@ -409,6 +409,17 @@ int glm52_selftest_mfma_layout(float* out, hipStream_t stream);
  * launches.  No counterpart in the reference: it shows how the items are dealt. */
 int glm52_debug_item_trace(void* buf, int64_t bytes);
 
+/* The set of item counters that the calling thread's last prefill tile launch deals from
+ * (-1: none yet).  A tile launch shares its items out between its workgroups through a set of
+ * counters in device memory, so launches in flight at once must not share a set.  Each kind of
+ * launch (gated; plain; o_proj and the atomic merge) at each block size has 1024 sets, which its
+ * launches outside graph capture take in turn, whatever their streams and threads (0 .. 1023),
+ * and 1024 more for captured launches (1024 .. 2047), which a graph keeps for its replays.  So:
+ * a stream may be at most 1023 launches of one kind ahead of another stream's launch that has
+ * not finished, and replays must not overlap if they are of one graph, or of graphs with 1024
+ * or more captured launches of one kind between them. */
+int glm52_debug_item_set(void);
+
 #ifdef __cplusplus
 }
 #endif

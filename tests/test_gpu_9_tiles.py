@@ -10,6 +10,7 @@ from __future__ import annotations
 import pytest
 import torch
 
+from fusion_amd import _lib
 from fusion_amd.dispatch import moe_align_block_size
 from fusion_amd.kernels import moe_gateup as KG
 from fusion_amd.kernels import oproj_resadd as KO
@@ -90,3 +91,118 @@ def test_oproj_tile_edges(gpu, M, K, N):
         acc = torch.ones(M, N, device=gpu)
         KO.gemm_launch(a, b, acc, res, {}, res is not None, True)
         _close(acc, 1 + (want if res is None else want + r.float()), K)
+
+
+def _side_by_side(pairs):
+    """Each pair of launches first in order, then at once on two streams, their outputs filled
+    with NaN: the same bits, from different sets of item counters."""
+    gate, s1, s2 = torch.cuda.Stream(), torch.cuda.Stream(), torch.cuda.Stream()
+    for name, (run_a, out_a), (run_b, out_b) in pairs:
+        print(f"two streams: {name}", flush=True)
+        want = []
+        for run, out in ((run_a, out_a), (run_b, out_b)):
+            out.fill_(float("nan"))
+            run()
+            torch.cuda.synchronize()
+            want.append(out.clone())
+            assert not bool(out.isnan().any()), name
+        for _ in range(3):
+            out_a.fill_(float("nan"))
+            out_b.fill_(float("nan"))
+            torch.cuda.synchronize()
+            sets = []
+            with torch.cuda.stream(gate):
+                torch.cuda._sleep(1_000_000)  # both launches wait for it, then start together
+                go = gate.record_event()
+            for s, run in ((s1, run_a), (s2, run_b)):
+                with torch.cuda.stream(s):
+                    s.wait_event(go)
+                    run()
+                    sets.append(_lib.query("glm52_debug_item_set"))
+            torch.cuda.synchronize()
+            assert torch.equal(out_a, want[0]) and torch.equal(out_b, want[1]), name
+            assert sets[0] != sets[1], (name, sets)
+
+
+@pytest.mark.parametrize("bm", [64, 128, 256])
+def test_two_streams_expert_gemms(gpu, bm):
+    """Instances that share a counter array, at once: packed unweighted and packed weighted,
+    and packed and in place."""
+    g = torch.Generator(device=gpu).manual_seed(bm)
+    E, N, K, T = 8, 1024, 1024, 2000
+    ids = torch.randint(0, E, (T, 1), generator=g, dtype=torch.int32, device=gpu)
+    a = torch.empty(T, K, dtype=BF16, device=gpu).normal_(0, 1, generator=g)
+    w = torch.empty(E, N, K, dtype=BF16, device=gpu).normal_(0, 0.02, generator=g)
+    wp, tw = KG.pack_w512(w, N, 0, False), torch.rand(T, generator=g, device=gpu)
+    sti, eids, ntp = moe_align_block_size(ids, bm, E)
+    o = [torch.empty(T, N, dtype=BF16, device=gpu) for _ in range(2)]
+    cfg = {"BLOCK_M": bm}
+
+    def packed(out, weights):
+        return lambda: KG.moe_gemm_packed(a, 1, wp, out, weights, sti, eids, ntp, T, N, False, cfg)
+
+    def in_place(out):
+        return lambda: KG.moe_gemm(a, 1, w, out, None, sti, eids, ntp, T, N, 0, False, cfg)
+
+    _side_by_side([("unweighted, weighted", (packed(o[0], None), o[0]), (packed(o[1], tw), o[1])),
+                   ("packed, in place", (packed(o[0], None), o[0]), (in_place(o[1]), o[1]))])
+
+
+def test_two_streams_oproj(gpu):
+    """o_proj with K slices (epilogue 3) beside o_proj without (epilogue 1, and 2 into fp32)."""
+    K, N = 4096, 1536
+    g = torch.Generator(device=gpu).manual_seed(3)
+    b = torch.empty(K, N, dtype=BF16, device=gpu).normal_(0, 0.02, generator=g)
+    assert _lib.query("glm52_oproj_splits", 256, N, K) > 1
+    assert _lib.query("glm52_oproj_splits", 12288, N, K) == 1
+
+    def chain(M, f32):
+        a = torch.empty(M, K, dtype=BF16, device=gpu).normal_(0, 1, generator=g)
+        r = torch.empty(M, N, dtype=BF16, device=gpu).normal_(0, 1, generator=g)
+        c = torch.empty(M, N, dtype=torch.float32 if f32 else BF16, device=gpu)
+
+        def run():
+            if f32:
+                c.zero_()
+            KO.gemm_launch(a, b, c, r, {}, True, f32)
+
+        return run, c
+
+    sliced, whole, whole32 = chain(256, False), chain(12288, False), chain(12288, True)
+    _side_by_side([("K slices, whole K", sliced, whole), ("whole K, K slices", whole, sliced),
+                   ("whole K, whole K into fp32", whole, whole32)])
+
+
+def test_captured_launches_keep_sets_of_their_own(gpu):
+    """A captured launch's counters are not among those that eager launches take in turn, so
+    replays run beside any number of eager launches; every replay gives the eager bits."""
+    g = torch.Generator(device=gpu).manual_seed(5)
+    E, N, K, T, bm = 4, 512, 256, 300, 64
+    ids = torch.randint(0, E, (T, 1), generator=g, dtype=torch.int32, device=gpu)
+    a = torch.empty(T, K, dtype=BF16, device=gpu).normal_(0, 1, generator=g)
+    wp = KG.pack_w512(torch.empty(E, N, K, dtype=BF16, device=gpu).normal_(0, 0.02, generator=g),
+                      N, 0, False)
+    lay = moe_align_block_size(ids, bm, E)
+    out, eager = (torch.empty(T, N, dtype=BF16, device=gpu) for _ in range(2))
+
+    def run(c):
+        KG.moe_gemm_packed(a, 1, wp, c, None, *lay, T, N, False, {"BLOCK_M": bm})
+        return _lib.query("glm52_debug_item_set")
+
+    assert run(eager) < 1024
+    torch.cuda.synchronize()
+    want = eager.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        sets = [run(out), run(out)]
+    assert min(sets) >= 1024 and sets[0] != sets[1]
+    side = torch.cuda.Stream()
+    for i in range(4):
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            for _ in range(300):  # 1200 in all: every eager set is taken once
+                assert run(eager) < 1024
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(eager, want), f"replay {i}"
