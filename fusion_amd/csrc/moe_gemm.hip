@@ -374,8 +374,8 @@ int a_bytes(int num_valid, int a_div, int64_t sa, int k) {
 // stream mapping (1) for what it does not cover (k % 512 != 0, output rows not 8-byte
 // aligned); block_m 64, 128 and 256 run the prefill tiles (5), and
 // at 64 and 128 the 256-row wide mapping (3) for what those do not cover (gated n_out %
-// 256 != 0, plain n_out % 512 != 0, token rows past 2^31 bytes); any other block_m (32)
-// runs the tiled mapping (2).  1 = stream, 2 = tiled, 3 = wide (64-k stages), 5 = prefill
+// 256 != 0, plain n_out % 512 != 0, token rows past 2^31 bytes, one expert's W rows past 2^32
+// bytes); any other block_m (32) runs the tiled mapping (2).  1 = stream, 2 = tiled, 3 = wide (64-k stages), 5 = prefill
 // tiles (moe_gemm_tile.h), 6 = contiguous-run weight stream (moe_gemm_runs.hip; block_m
 // 16) force one mapping.
 extern "C" int glm52_moe_gemm(const void* a, int64_t stride_am, int a_row_div, const void* w,
@@ -402,8 +402,8 @@ extern "C" int glm52_moe_gemm(const void* a, int64_t stride_am, int a_row_div, c
   const bool weighted = topk_weights != nullptr;
   const bool auto_wide = variant == 0 && (block_m == 64 || block_m == 128 || block_m == 256);
   if (variant == 5 || auto_wide) {
-    // the tiles address token rows with 32-bit byte offsets; shapes they have no
-    // instance for fall back to the 256-row mapping when the mapping was not forced
+    // the tiles address token rows and an expert's W rows with 32-bit byte offsets; shapes
+    // they have no instance for fall back to the 256-row mapping when the mapping was not forced
     const int rc = g.a_bytes < 0x7ffffff0 ? launch_tile(g, capacity, gated != 0, weighted, stream)
                                           : GLM52_EUNSUPPORTED;
     if (rc != GLM52_EUNSUPPORTED || variant == 5) return rc;

@@ -18,6 +18,14 @@ constexpr uint32_t kTokenBytes = 0x7ffffff0u;  // descriptor size of the token r
 constexpr uint32_t kInPlaceBytes = 0xfffffff0u;  // descriptor size of one expert's row-major W
 constexpr uint32_t kNowhere = 0x90000000u;     // lane offset of a padding row: past kTokenBytes
 
+// Whether one expert's row-major W rows -- 0 .. n_out - 1, and with gate_up > 0 those from
+// gate_up on as well, k elements each at a stride of swn -- fit the descriptor, so that no
+// lane's 32-bit offset wraps.
+inline bool in_place_fits(int gate_up, int n_out, int64_t swn, int k) {
+  return swn >= 0 &&
+         (((int64_t)gate_up + n_out - 1) * swn + k) * 2 <= (int64_t)kInPlaceBytes;
+}
+
 // Stage s of nk (the item's first stage is krot, wrapping; `step` bytes from one stage to the
 // next) of an operand of `bytes` bytes: the descriptor size and the scalar offsets of the stage
 // and, where two are loaded together (nk, s and krot even, step 64), of the one after it.  The

@@ -12,6 +12,7 @@ import torch
 
 from fusion_amd import _lib
 from fusion_amd.dispatch import moe_align_block_size
+from fusion_amd.kernels import moe_down_merge as KD
 from fusion_amd.kernels import moe_gateup as KG
 from fusion_amd.kernels import oproj_resadd as KO
 
@@ -206,3 +207,51 @@ def test_captured_launches_keep_sets_of_their_own(gpu):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want) and torch.equal(eager, want), f"replay {i}"
+
+
+@pytest.mark.parametrize("gated", [False, True])
+def test_weight_rows_past_4_gib(gpu, gated):
+    """Row-major W as a view with a row pitch of 8 MB, one expert spanning more than 2^32 bytes:
+    64- and 128-token blocks give the rows' results, 256-token blocks and the atomic merge
+    refuse it; a span just inside runs the tiles with the contiguous copy's bits."""
+    E, N, K, T = 2, 512, 256, 200
+    inside = ((0xfffffff0 // 2 - K) // (N - 1)) // 8 * 8
+    pitch = inside + 8
+    g = torch.Generator(device=gpu).manual_seed(9)
+    vals = torch.empty(E, N, K, dtype=BF16, device=gpu).normal_(0, 1, generator=g).clamp_(-2, 2)
+    big = torch.empty(N * pitch, dtype=BF16, device=gpu)
+    ids = torch.randint(0, E, (T, 1), generator=g, dtype=torch.int32, device=gpu)
+    a = torch.empty(T, K, dtype=BF16, device=gpu).normal_(0, 1, generator=g).clamp_(-2, 2)
+    full = torch.stack([vals[int(e)].float() @ x.float() for e, x in zip(ids.view(-1), a)])
+    n_out = N // 2 if gated else N
+    want = torch.nn.functional.silu(full[:, :n_out]) * full[:, n_out:] if gated else full
+    for bm in (64, 128, 256):
+        print(f"weight span bm={bm} gated={gated}", flush=True)
+        lay = moe_align_block_size(ids, bm, E)
+
+        def run(w):
+            c = torch.full((T, n_out), float("nan"), dtype=BF16, device=gpu)
+            KG.moe_gemm(a, 1, w, c, None, *lay, T, n_out, n_out if gated else 0, gated,
+                        {"BLOCK_M": bm})
+            return c
+
+        ref = run(vals)
+        w_in = big.as_strided((E, N, K), (K, inside, 1))
+        w_in.copy_(vals)
+        assert torch.equal(run(w_in), ref)
+        w_past = big.as_strided((E, N, K), (K, pitch, 1))
+        w_past.copy_(vals)
+        if bm == 256:
+            with pytest.raises(RuntimeError, match="unsupported"):
+                run(w_past)
+        elif gated:  # silu's slope is at most 1.1: the sums' errors reach the product twice
+            err = (run(w_past).float() - want).abs()
+            tol = want.abs() * 2.0 ** -7 + (full[:, :n_out].abs() + 1.1 * full[:, n_out:].abs()
+                                            + 1) * K * 4 * 2.0 ** -22
+            assert bool((err <= tol).all())
+        else:
+            _close(run(w_past), full, K)
+            out = torch.zeros(T, N, dtype=BF16, device=gpu)
+            with pytest.raises(RuntimeError, match="unsupported"):
+                KD.launch_down(a, w_past, out, torch.ones(T, device=gpu), *lay, T, 1,
+                               {"BLOCK_M": bm}, True)
