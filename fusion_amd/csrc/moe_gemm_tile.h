@@ -34,9 +34,9 @@
 //
 // Order and dealing.  The kernel is persistent, one workgroup per CU.  Expert-aligned contiguous
 // shares per XCD, dealt from per-XCD counters; the row blocks of an expert in groups of
-// kRowGroup, so that the 32 workgroups of an XCD read 4 row blocks and 8 column tiles at a
-// time (12 operand tiles for 32 products; column tile by column tile it was 33: o_proj at
-// M = 8192 1941 -> 1352 us with nothing else changed).
+// kRowGroup, so that the 32 workgroups of an XCD read 4 row blocks and 8 column tiles (or 8
+// and 4) at a time (12 operand tiles for 32 products; column tile by column tile it was 33:
+// o_proj at M = 8192 1941 -> 1352 us with nothing else changed).
 //
 // Between items.  The next item is decoded and its first five stages are issued before the
 // current item's epilogue, so their latency runs under it.
@@ -54,7 +54,6 @@ namespace {  // one copy per source file: each has its own counters and their se
 // the kernel's lambdas share its state by reference, which stays in registers only inlined
 #define GLM52_INLINE __attribute__((always_inline))
 
-constexpr int kRowGroup = 4;
 constexpr int kBK = 32;  // k per stage
 
 // Counters the items are dealt from, a set per launch: XCD x's at 16 x, the exits at 128; the
@@ -161,6 +160,12 @@ __global__ __launch_bounds__(256) void moe_gemm_tile_kernel(GemmArgs p) {
   constexpr int kWI = NT / 64;  // W load instructions per wave and stage
   constexpr int kAI = MT / 64;  // token-row load instructions per wave and stage
   constexpr int kQ = MT / kWave;
+  // Row blocks of an expert per group of the item order.  An XCD's 32 workgroups read 12 operand
+  // tiles at a time with groups of 4 (4 row blocks and 8 column tiles) and of 8 alike.  In o_proj
+  // 8 stream B once, not twice, for 5 to 8 row blocks (M = 1536 369 -> 348 us, M = 2048 379 ->
+  // 362; M = 8192 1278 -> 1272).  The expert GEMMs stay at 4: the T = 8192 block is the same
+  // with 8 (6025, 5970 us, runs 1 % apart), and two of three blocks at T = 3000 - 4096 2-3 % slower.
+  constexpr int kRowGroup = PACKED && !GATED && !WEIGHTED ? 8 : 4;
   const unsigned long long t_start = p.wg_trace ? __builtin_amdgcn_s_memrealtime() : 0ull;
   int n_run = 0;  // items this workgroup ran (the trace record)
   constexpr int NO = GATED ? NT / 2 : NT;    // outputs per tile; a packed tile has twice those
