@@ -291,25 +291,35 @@ Split decode_split(int M, int N, int K) {
   return sp;
 }
 
-// Rows per tile of the prefill mapping: the 256 x 256 tile from 256 rows (it stages a fifth
-// fewer bytes through LDS per flop than 128 rows x 512 columns: o_proj at M = 256 188 -> 148
-// us, at M = 2048 483 -> 458 us, and at M = 8192, once an XCD's workgroups took 4 row blocks x
-// 8 column tiles at a time, 1642 -> 1352 us), else 128 rows, or 64 where they hold
-// every row (with its 256-row tiles, M = 64: 85 -> 75 us).
-int prefill_bm(int M) { return M >= 256 ? 256 : M > 64 ? 128 : 64; }
+// Tiles of the prefill mapping with bm rows and 256 columns each.
+int64_t prefill_items(int M, int N, int bm) { return (int64_t)((M + bm - 1) / bm) * (N / 256); }
 
-// K slices of the prefill mapping: enough (1 .. 16, powers of two) to give the 256 CUs
-// about one tile each, keeping every slice a multiple of 64 and at least 1024 k.
-int prefill_splits(int M, int N, int K) {
-  const int bm = prefill_bm(M);
-  const int64_t items = (int64_t)((M + bm - 1) / bm) * (N / 256);
+// K slices over `items` tiles: enough (1 .. 16, powers of two) to give the 256 CUs about one
+// each, keeping every slice a multiple of 64 and at least 1024 k.
+int k_slices(int64_t items, int K) {
   int S = 1;
   while (S < 16 && items * S * 2 <= 256 && K % (64 * S * 2) == 0 && K / (S * 2) >= 1024) S *= 2;
   return S;
 }
 
-int64_t layout_bytes(int M, int S) {
-  const int bm = prefill_bm(M);
+// Rows per tile of the prefill mapping: from 256 rows the 256 x 256 tile (it stages a fifth
+// fewer bytes through LDS per flop than 128 rows x 512 columns: o_proj at M = 256 188 -> 148
+// us, at M = 2048 483 -> 458 us, and at M = 8192, once an XCD's workgroups took 4 row blocks x
+// 8 column tiles at a time, 1642 -> 1352 us), unless 128 rows over the same K slices still
+// give every tile a CU of its own: each then takes as many stages of about half the time
+// (K = 32768: M = 513 378 -> 236 us, M = 640 379 -> 255; with more stages or a second round they
+// lose, M = 512 227 -> 243 and M = 768 382 -> 454).  Below 256 rows 128, or 64 where they hold
+// every row (with its 256-row tiles, M = 64: 85 -> 75 us).
+int prefill_bm(int M, int N, int K) {
+  if (M < 256) return M > 64 ? 128 : 64;
+  return prefill_items(M, N, 128) * k_slices(prefill_items(M, N, 256), K) <= 256 ? 128 : 256;
+}
+
+int prefill_splits(int M, int N, int K) {
+  return k_slices(prefill_items(M, N, prefill_bm(M, N, K)), K);
+}
+
+int64_t layout_bytes(int M, int bm, int S) {
   const int64_t per = ((int64_t)M + bm - 1) / bm * bm;
   const int64_t cap = per * S;
   return (cap + cap / bm + 1 + 64) * 4;
@@ -326,7 +336,8 @@ extern "C" int64_t glm52_oproj_workspace_bytes(int M, int N, int K) {
   const Split sp = decode_split(M, N, K);
   const int64_t dec = M <= 16 ? (int64_t)sp.S * M * N * 4 : 0;
   const int S = prefill_splits(M, N, K);
-  const int64_t pre = round256(layout_bytes(M, S)) + (S > 1 ? (int64_t)M * S * N * 4 : 0);
+  const int64_t pre = round256(layout_bytes(M, prefill_bm(M, N, K), S)) +
+                      (S > 1 ? (int64_t)M * S * N * 4 : 0);
   return (dec > pre ? dec : pre) + 256;
 }
 
@@ -396,17 +407,18 @@ extern "C" int glm52_oproj_gemm(const void* a, int64_t stride_am, const void* b,
   const int S = splits;
   if (S < 1 || (N % 512) || (K % (64 * S))) return GLM52_EUNSUPPORTED;
   if (S > 1 && stride_am != K) return GLM52_EINVAL;  // A is viewed as [M S, K / S]
-  if (workspace_bytes < round256(layout_bytes(M, S)) + (S > 1 ? (int64_t)M * S * N * 4 : 0))
+  const int BM = prefill_bm(M, N, K);
+  if (workspace_bytes < round256(layout_bytes(M, BM, S)) + (S > 1 ? (int64_t)M * S * N * 4 : 0))
     return GLM52_EINVAL;
   const int Ks = K / S;
   // one "expert" per K slice over the split row layout, written into the workspace
-  const int BM = prefill_bm(M);
   const int per = (M + BM - 1) / BM * BM;
   const int cap = per * S;
   int32_t* sti = static_cast<int32_t*>(workspace);
   int32_t* eids = sti + cap;
   int32_t* ntp = eids + cap / BM + 16;
-  float* part = reinterpret_cast<float*>(static_cast<char*>(workspace) + round256(layout_bytes(M, S)));
+  float* part = reinterpret_cast<float*>(static_cast<char*>(workspace) +
+                                         round256(layout_bytes(M, BM, S)));
   split_layout_kernel<<<(cap + 255) / 256 < 1024 ? (cap + 255) / 256 : 1024, 256, 0, stream>>>(
       M, S, BM, per, sti, eids, ntp);
   hipError_t err = hipGetLastError();

@@ -75,7 +75,12 @@ def test_tile_edges(gpu, rows, K, bm):
 
 @pytest.mark.parametrize("M,K,N", [(17, 64, 512), (64, 2048, 512), (65, 1024, 1536),
                                    (200, 4160, 512), (256, 64, 512), (257, 1024, 1024), (700, 2112, 512),
-                                   (2300, 512, 1536)])
+                                   (2300, 512, 1536),
+                                   # 256-row tiles: one K slice, and four (N = 6144)
+                                   (1281, 64, 6144), (2300, 128, 6144), (257, 4096, 6144),
+                                   (383, 4096, 6144), (512, 4096, 6144),
+                                   # 128-row tiles past 256 rows, two K slices; 256-row tiles again
+                                   (513, 2048, 6144), (640, 2048, 6144), (641, 2048, 6144)])
 def test_oproj_tile_edges(gpu, M, K, N):
     """o_proj from 17 rows: every epilogue, K slices or none, ragged last blocks, and row
     blocks past one order group."""
