@@ -623,10 +623,15 @@ __global__ __launch_bounds__(256) void moe_gemm_tile_kernel(GemmArgs p) {
       }
     };
     // An instance per 16-token group count, or per even one: a part-filled block then
-    // multiplies up to 32 token rows of padding more.  The odd counts are kept where the matrix
-    // cores and the power limit weigh most, the 256-token expert GEMMs (T = 8192 block 6148 ->
-    // 6074 us).  With them the 64- and 128-token tiles, which wait for their weights, and
-    // o_proj lose (T = 1333 block 3222 -> 3313 us, o_proj at M = 256 131 -> 167 us).
+    // multiplies up to 32 token rows of padding more.  Every count at 256 tokens with a bf16
+    // store (the expert GEMMs, and o_proj without residual or K slices), where the matrix cores
+    // and the power limit weigh most (T = 8192 block 6148 -> 6074 us).  With the odd counts the
+    // 64- and 128-token tiles, which wait for their weights, and the other epilogues lose (T =
+    // 1333 block 3222 -> 3313 us, o_proj at M = 256 131 -> 167 us, at M = 8192 1305 -> 1344).
+    // o_proj's K slices at 256 rows have two instances only, 2 and 8: a tile's items all run at
+    // once there, so a shorter last block ends no sooner, and its pace parts from that of the
+    // block it shares W with (K = 32768: M = 400 226 -> 219 us, M = 256 139 -> 135; M = 300 216.5
+    // -> 222; K = 16384: M = 700 202 -> 189).
     const int nvg = (c_nv + 16 * kWaveM - 1) / (16 * kWaveM);  // 16-token groups per wave
     auto pick = [&](auto nt) GLM52_INLINE {
       constexpr int MAXV = MT / (16 * kWaveM);
@@ -641,6 +646,7 @@ __global__ __launch_bounds__(256) void moe_gemm_tile_kernel(GemmArgs p) {
         });
         if (!done) run(std::integral_constant<int, MAXV>{}, nt);
       } else if (MAXV == 2 || nvg <= 2) run(std::integral_constant<int, 2>{}, nt);
+      else if constexpr (MAXV == 8 && EPI == 3) run(std::integral_constant<int, MAXV>{}, nt);
       else if (MAXV == 4 || nvg <= 4) run(std::integral_constant<int, MAXV < 4 ? 2 : 4>{}, nt);
       else if constexpr (MAXV == 8) {
         if (nvg <= 6) run(std::integral_constant<int, 6>{}, nt);
