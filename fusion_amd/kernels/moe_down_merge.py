@@ -21,13 +21,15 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
-from .moe_gateup import check_layout, moe_gemm
+from .moe_gateup import check_layout, moe_gemm, tile_smem_bytes
 
 
 def smem_bytes(cfg: dict) -> int:
     bm = cfg["BLOCK_M"]
     if bm == 16 or cfg.get("variant") == "stream":
         return 4096
+    if bm in (64, 128, 256) and cfg.get("variant") in (None, "auto", "w512"):
+        return tile_smem_bytes(bm, 512 if bm < 256 and cfg.get("w2_packed") is not None else 256)
     return 2 * (bm + 128) * (64 + 8) * 2 + 4 * bm
 
 

@@ -201,16 +201,23 @@ def moe_gemm_shared(a, a_row_div, w, c, topk_weights, sorted_token_ids, expert_i
     )
 
 
+def tile_smem_bytes(bm: int, w_rows: int) -> int:
+    """LDS of a prefill tile of `bm` tokens x `w_rows` W rows: as many 32-k stages as 160 KB
+    hold.  W in place has 256 rows, the packed expert GEMMs 512 at 64 and 128 tokens."""
+    stage = (w_rows + bm) * 32 * 2
+    return 163840 // stage * stage
+
+
 def smem_bytes(cfg: dict, fused: bool) -> int:
     """LDS bytes of the mapping this cfg selects (`moe_gateup.smem_bytes`'s question)."""
     bm = cfg["BLOCK_M"]
     variant = cfg.get("variant")
-    if variant == "runs" or (variant is None and bm == 16):
+    if variant == "runs" or (variant in (None, "auto") and bm == 16):
         return 4 * 32 * 512 * 2 + 4 * 4 * 64 * 4
     if variant == "stream":
         return 8192
-    if variant == "w512" or (variant is None and bm in (64, 128, 256)):
-        return 5 * (256 + bm) * 32 * 2 if bm == 256 else 4 * (512 + bm) * 32 * 2
+    if variant == "w512" or (variant in (None, "auto") and bm in (64, 128, 256)):
+        return tile_smem_bytes(bm, 256)
     if variant == "wide":
         return 3 * (256 + bm) * 64 * 2 + 4 * bm
     nb = 128
