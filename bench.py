@@ -477,7 +477,7 @@ def down_merge_bench(blk, W, T: int, n_e: int, timed, steps: int, warmup: int) -
     H, I, k = blk.H, blk.I, blk.topk
     R = T * k
     cfg = {"BLOCK_M": blk.bm}
-    if blk.packed and blk.bm != 16:  # the 512-row mapping of the atomic merge reads it
+    if blk.packed and blk.bm != 16:  # the prefill tiles of the atomic merge read it
         cfg["w2_packed"] = blk.experts.w2
     tw = blk.topw.reshape(-1)
     c3 = torch.empty(R, H, dtype=torch.bfloat16, device=blk.h.device)

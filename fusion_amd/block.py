@@ -218,7 +218,7 @@ class MoEBlock:
         self.cfg_topk = {"correction_bias": bias, "scale": scale, "workspace": self.router_ws}
         self.graph = None
         # the GEMMs read the packed layout at every block size (16: the weight stream over
-        # load slots; 64, 128, 256: the 512-row and 256-row tiles)
+        # load slots; 64, 128, 256: the prefill tiles)
         self.packed = self.experts is not None
         if self.packed and not (self.shared_fused or (self.bm in (64, 128, 256)
                                                       and self.sbm in (64, 128, 256))):

@@ -3,7 +3,8 @@
 // Conventions used by every kernel in this library:
 //   * bf16 tensors are passed as `const uint16_t*` and converted with the helpers
 //     below; fp32 -> bf16 is round-to-nearest-even with NaN mapped to 0x7fc0, which is
-//     the rounding torch's `.to(torch.bfloat16)` applies.
+//     the rounding torch's `.to(torch.bfloat16)` applies (the grouped GEMM tiles use the
+//     hardware's conversion: the same values, a NaN as 0xffc0).
 //   * 16-byte (8 x bf16) vector accesses use `uint4`; callers guarantee 16-byte
 //     alignment of the base pointers and of every row stride they pass.
 //   * Every launch goes on the caller's stream and nothing here allocates memory.

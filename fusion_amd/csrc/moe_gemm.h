@@ -213,8 +213,7 @@ int note_item_set(int set);
 // rows n and the `up` rows gate_up_offset + n), K = k.  Returns the bytes written, or a
 // negative error for a shape the packed layout does not hold (out = null: size only).
 int64_t pack_w512(const uint16_t* w, int64_t swe, int64_t swn, int E, int n_out, int k,
-                     int gate_up_offset, bool gated, uint16_t* out, hipStream_t st,
-                     int64_t swk = 1);
+                  int gate_up_offset, bool gated, uint16_t* out, hipStream_t st, int64_t swk = 1);
 
 // The decode mapping that streams W as contiguous 1 KB row runs (moe_gemm_runs.hip): block
 // size 16; an optional extra expert (x_rows > 0) as in the stream mapping; `route`: the

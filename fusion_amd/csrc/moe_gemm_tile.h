@@ -32,14 +32,15 @@
 // token rows and shared tiles that other workgroups of the XCD re-read from L2 (T = 8192 with
 // skewed load: w13 3737 -> 3580 us).
 //
-// Order and dealing.  The kernel is persistent, one workgroup per CU.  Expert-aligned contiguous
-// shares per XCD, dealt from per-XCD counters; the row blocks of an expert in groups of
+// Order and dealing.  The kernel is persistent, one workgroup per CU.  Each XCD owns a contiguous
+// share of the items, ordered expert by expert (a share may end inside an expert), and deals it
+// from a counter of its own, then helps the other XCDs; the row blocks of an expert in groups of
 // kRowGroup, so that the 32 workgroups of an XCD read 4 row blocks and 8 column tiles (or 8
 // and 4) at a time (12 operand tiles for 32 products; column tile by column tile it was 33:
 // o_proj at M = 8192 1941 -> 1352 us with nothing else changed).
 //
-// Between items.  The next item is decoded and its first five stages are issued before the
-// current item's epilogue, so their latency runs under it.
+// Between items.  The next item is decoded and the first stages that fill its ring (four to
+// eight) are issued before the current item's epilogue, so their latency runs under it.
 #pragma once
 
 #include "moe_gemm.h"
@@ -122,7 +123,7 @@ GLM52_DEV void dma16b(const u32x4_t& srd, uint32_t voff, uint32_t soff, uint32_t
                  : "memory");
 }
 
-// Two fp32 as packed bf16, round to nearest even.
+// Two fp32 as packed bf16, round to nearest even, as pack8 but for a NaN's bits (0xffc0 here).
 GLM52_DEV uint32_t cvt_pk_bf16(float lo, float hi) {
   uint32_t r;
   asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(lo), "v"(hi));

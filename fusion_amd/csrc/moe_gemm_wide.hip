@@ -29,7 +29,6 @@
 // once and served to the others from the XCD's L2.
 #include "moe_gemm.h"
 
-#include <atomic>
 #include <type_traits>
 
 using namespace glm52;

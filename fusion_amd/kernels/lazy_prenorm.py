@@ -48,7 +48,7 @@ def fold_weight_nk(bt: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 def smem_bytes(cfg: dict) -> int:
     """LDS of the consumers that run: the router's token tile (74752 B) and the grouped
-    GEMM's 512-row ring (163840 B); the rstd pass uses none."""
+    GEMM's tile ring (at most 163840 B); the rstd pass uses none."""
     return 163840
 
 

@@ -39,7 +39,7 @@ def launch_down(a, w2, c, topk_weights_flat, sorted_token_ids, expert_ids,
     c: [rows, H] when fuse_merge=False, else the pre-seeded [T, H] output, to which every
     routed row's bf16 result is added with packed bf16 atomics (`moe_down_merge.py:
     160-169`); `cfg["w2_packed"]` (`moe_gateup.pack_w512(w2, H, 0, False)`) may supply
-    the packed weights the 64/128-row mapping reads."""
+    the packed weights the prefill tiles (BLOCK_M 64, 128, 256) read."""
     if not fuse_merge:
         moe_gemm(a, 1, w2, c, topk_weights_flat, sorted_token_ids, expert_ids,
                  num_tokens_post_padded, num_valid_tokens, w2.shape[1], 0, False, cfg)

@@ -13,12 +13,12 @@ conventions (`glm52/kernels/REFERENCES.md:41-51`): A rows are gathered with
 `cfg["BLOCK_M"]` must equal the layout's block size (checked).  `cfg["variant"]` may
 force "stream" (weight-streaming decode mapping), "tiled" (register-staged LDS tiles),
 "wide" (256-row W tiles fed by direct global -> LDS loads through 64-k stages), "w512"
-(512-row W tiles on the 32x32x16 MFMA, 32-k stages; 256 x 256 tiles at BM = 256) or
+(the prefill tiles on the 16x16x32 MFMA, 32-k stages; 512 or 256 W rows) or
 "runs" (the decode weight stream read as contiguous 1 KB row runs through LDS).  By
 default BM = 16 runs "runs", and "stream" for the shapes it does not cover (K % 512 != 0,
 output rows not 8-byte aligned); BM in {64, 128, 256} runs "w512", and at 64 and 128
-"wide" for the shapes it does not cover (gated N % 256 != 0, plain N % 512 != 0); any
-other BM (32) runs "tiled".
+"wide" for the shapes it does not cover (gated N % 256 != 0, plain N % 512 != 0, A past
+2^31 bytes, one expert's W rows past 2^32); any other BM (32) runs "tiled".
 """
 
 from __future__ import annotations
@@ -107,7 +107,7 @@ def check_packed(w_packed, n_out: int, K: int, gated: bool) -> None:
 
 def moe_gemm_packed(a, a_row_div, w_packed, c, topk_weights, sorted_token_ids, expert_ids,
                     num_tokens_post_padded, num_valid_tokens, n_out, gated, cfg):
-    """`moe_gemm` (BLOCK_M 64 or 128) on weights packed by `pack_w512`: the same bits."""
+    """`moe_gemm` (BLOCK_M 16, 64, 128 or 256) on weights packed by `pack_w512`: the same bits."""
     _lib.require_gpu(a, w_packed, c, sorted_token_ids, expert_ids, num_tokens_post_padded,
                      topk_weights)
     if a.dtype != torch.bfloat16 or w_packed.dtype != torch.bfloat16 or c.dtype != torch.bfloat16:

@@ -190,10 +190,11 @@ int glm52_moe_gemm_route_shared_packed(const float* logits, int64_t stride_l, co
  * topk_weights non-null = MUL_ROUTED_WEIGHT).  A rows are a[sorted_id / a_row_div],
  * W is [E, N, K] with K contiguous, C rows are indexed by the flat token id.
  * variant: 0 auto, 1 weight-streaming, 2 register-staged LDS tiles (block_m in {32, 64,
- * 128}), 3 / 4 wide 256-row W tiles fed by direct global -> LDS loads through 64-k / 32-k
- * stages (block_m in {64, 128}), 5 512-row W tiles on the 32x32x16 MFMA (block_m in
- * {64, 128}), 6 contiguous-run weight stream (block_m 16); auto runs 6 at block_m 16 and
- * 5 at 64 and 128, falling back to 1 and 3 for shapes those have no instance for. */
+ * 128}), 3 wide 256-row W tiles fed by direct global -> LDS loads through 64-k stages
+ * (block_m in {64, 128}), 5 the prefill tiles (block_m in {64, 128, 256}; gated n_out % 256 ==
+ * 0, plain n_out % 512 == 0, A's rows within 2^31 bytes, one expert's W rows within 2^32), 6
+ * contiguous-run weight stream (block_m 16); auto runs 6 at block_m 16 and 5 at 64, 128 and
+ * 256, falling back to 1 at 16 and to 3 at 64 and 128 for shapes those have no instance for. */
 int glm52_moe_gemm(const void* a, int64_t stride_am, int a_row_div, const void* w,
                    int64_t stride_we, int64_t stride_wn, int gate_up_offset, void* c,
                    int64_t stride_cm, const float* topk_weights, const int32_t* sorted_token_ids,
@@ -216,9 +217,9 @@ int glm52_moe_gemm_shared(const void* a, int64_t stride_am, int a_row_div, const
                           int shared_rows, int n_out, int k, int gated, hipStream_t stream);
 
 /* Packed weights, the one resident layout of this build's block: no counterpart in the
- * reference, whose kernels read W in place.  The prefill mapping reads each 32-k stage of a
- * 512-row W tile as 512 runs of 64 bytes; the packed copy holds every stage as 32 KB of
- * contiguous memory in the order the tile's loads fill LDS, and each 1 KB load slot of a
+ * reference, whose kernels read W in place.  In place the prefill tiles read W as runs of 128
+ * bytes, one per row and pair of 32-k stages; the packed copy holds every stage of 512 rows as
+ * 32 KB of contiguous memory in the order the tile's loads fill LDS, and each 1 KB load slot of a
  * stage (16 rows x 32 k) is also what the decode weight stream reads.  Packing is done once
  * per weight tensor; the GEMMs on the packed copy compute the same bits as glm52_moe_gemm
  * (variants 5 and 6) on the original.
@@ -264,8 +265,8 @@ int glm52_moe_gemm_packed_shared(const void* a, int64_t stride_am, int a_row_div
  *     with B N-contiguous streams B (split K, fixed-order reduction); otherwise b_packed
  *     from glm52_oproj_pack is required (N % 512 == 0, K % 64 == 0).  The workspace holds
  *     glm52_oproj_workspace_bytes(M, N, K) bytes.
- *   glm52_oproj_pack / glm52_oproj_packed_bytes: B packed once as the 512-row tile
- *     mapping's W = B^T, cut into `splits` K slices (no counterpart in the reference);
+ *   glm52_oproj_pack / glm52_oproj_packed_bytes: B packed once as the prefill tiles'
+ *     W = B^T, cut into `splits` K slices (no counterpart in the reference);
  *     glm52_oproj_splits(M, N, K) is the count glm52_oproj_gemm wants for that shape
  *     (more slices when M gives too few tiles to fill the GPU).
  *   glm52_cast_add: o = bf16(c (+ r)), c bf16 or fp32 -- oproj_resadd.epilogue_launch
@@ -322,8 +323,8 @@ int glm52_router_rstd(const void* y, int64_t stride_y, const void* wgt, int64_t 
  * FUSE_MERGE epilogue :160-169).  For every valid flat token f of the layout,
  * out[f / top_k, :] += bf16(topk_weights[f] * (a[f] . w[e]^T)), each add a packed bf16
  * atomic, so the rounding order depends on timing.  out [T, n_out] is seeded by the
- * caller (zeros or the residual; launch_seed).  block_m 16, 64 or 128; w_packed
- * (glm52_pack_w512, may be null; not with block_m 16) is read by the 64/128 mapping. */
+ * caller (zeros or the residual; launch_seed).  block_m 16, 64, 128 or 256; w_packed
+ * (glm52_pack_w512, may be null; not with block_m 16) is read by the prefill tiles. */
 int glm52_moe_down_merge(const void* a, int64_t stride_am, const void* w, int64_t stride_we,
                          int64_t stride_wn, const void* w_packed, void* out, int64_t stride_om,
                          const float* topk_weights, const int32_t* sorted_token_ids,
@@ -401,7 +402,7 @@ int glm52_stream_read(const void* buf, int64_t bytes, int nontemporal, int grid,
  * No counterpart in the reference. */
 int glm52_selftest_mfma_layout(float* out, hipStream_t stream);
 
-/* Measurement hook of the prefill tile (the 512-row and 256 x 256 tile launches of
+/* Measurement hook of the prefill tile (the launches at block_m 64, 128 and 256 of
  * glm52_moe_gemm, glm52_moe_gemm_packed(_shared), glm52_oproj_gemm): with `buf` set (at least
  * 256 x 4 words of device memory), every later launch writes, per workgroup w, words
  * 4w .. 4w+3 = its start and end on the 100 MHz wall clock, the items it ran and its XCD;
@@ -412,8 +413,8 @@ int glm52_debug_item_trace(void* buf, int64_t bytes);
 /* The set of item counters that the calling thread's last prefill tile launch deals from
  * (-1: none yet).  A tile launch shares its items out between its workgroups through a set of
  * counters in device memory, so launches in flight at once must not share a set.  Each kind of
- * launch (gated; plain; o_proj and the atomic merge) at each block size has 1024 sets, which its
- * launches outside graph capture take in turn, whatever their streams and threads (0 .. 1023),
+ * launch (gated; plain, o_proj without residual and K slices included; o_proj's others and the
+ * atomic merge) at each block size has 1024 sets, which its launches outside graph capture take in turn, whatever their streams and threads (0 .. 1023),
  * and 1024 more for captured launches (1024 .. 2047), which a graph keeps for its replays.  So:
  * a stream may be at most 1023 launches of one kind ahead of another stream's launch that has
  * not finished, and replays must not overlap if they are of one graph, or of graphs with 1024

@@ -578,11 +578,12 @@ def test_moe_gemm_packed_shared_matches_separate_launches(gpu, bm, T):
 @pytest.mark.parametrize("bm", [64, 128, 256])
 def test_w512_item_dealing(gpu, bm):
     """The prefill tile deals its items from per-XCD counters that the last workgroup out
-    clears, one counter set per launch out of 64 in turn.  (1) A layout block with no real
+    clears, one counter set per launch out of 1024 in turn.  (1) A layout block with no real
     row (the workgroup fetches the next item at once) leaves the results as they are
-    without it.  (2) 70 launches in a row (more than the 64 sets, so every set is reused
-    after it was cleared) all give the first launch's bits.  (3) Two launches issued on two
-    streams at once give the bits of the same launches in order."""
+    without it.  (2) 1030 launches in a row (more than the 1024 sets, so sets are reused
+    after they were cleared) all give the first launch's bits.  (3) Two launches issued on
+    two streams at once give the bits of the same launches in order (pairs that share a
+    counter array: test_gpu_9_tiles.py)."""
     say(f"w512 item dealing bm={bm}")
     T, E, H, I, k = 300, 8, 512, 256, 8
     a, w13, w2, ids, tw = _gemm_problem(T, E, H, I, k, 700 + bm, gpu)
@@ -623,7 +624,7 @@ def test_w512_item_dealing(gpu, bm):
 
     # (2) launches in a row, every output refilled first
     y3 = torch.empty_like(y)
-    for i in range(70):
+    for i in range(1030):
         y3.fill_(nan)
         down((sti, eids, ntp), act, y3)
         assert torch.equal(y3, y), f"launch {i}"

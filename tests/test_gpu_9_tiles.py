@@ -205,9 +205,10 @@ def test_captured_launches_keep_sets_of_their_own(gpu):
     side = torch.cuda.Stream()
     for i in range(4):
         out.fill_(float("nan"))
+        eager.fill_(float("nan"))
         torch.cuda.synchronize()
         with torch.cuda.stream(side):
-            for _ in range(300):  # 1200 in all: every eager set is taken once
+            for _ in range(300):  # 1200 in all: every eager set is taken
                 assert run(eager) < 1024
         graph.replay()
         torch.cuda.synchronize()
@@ -260,3 +261,55 @@ def test_weight_rows_past_4_gib(gpu, gated):
             with pytest.raises(RuntimeError, match="unsupported"):
                 KD.launch_down(a, w_past, out, torch.ones(T, device=gpu), *lay, T, 1,
                                {"BLOCK_M": bm}, True)
+
+
+@pytest.mark.parametrize("bm", [64, 128, 256])
+def test_nan_outputs(gpu, bm):
+    """A NaN of either sign in a token row or a weight row reaches that row's or column's
+    outputs and no other, in every bf16 store of the tiles."""
+    g = torch.Generator(device=gpu).manual_seed(bm)
+    E, N, K, T = 2, 512, 256, 300
+    ids = (torch.arange(T, device=gpu) % E).to(torch.int32).view(T, 1)
+    a = torch.empty(T, K, dtype=BF16, device=gpu).normal_(0, 1, generator=g)
+    w = torch.empty(E, N, K, dtype=BF16, device=gpu).normal_(0, 1, generator=g)
+    a.view(torch.int16)[[7, 130, 290], [3, 255, 64]] = torch.tensor(
+        [0x7F81, -1, 0x7FC0], dtype=torch.int16, device=gpu)
+    w.view(torch.int16)[1, [11, 300], 5] = torch.tensor([-63, 0x7FFF], dtype=torch.int16, device=gpu)
+    nan = torch.zeros(T, N, dtype=torch.bool, device=gpu)
+    nan[[7, 130, 290]] = True
+    nan[1::2, 11] = nan[1::2, 300] = True
+    lay = moe_align_block_size(ids, bm, E)
+    cfg, tw = {"BLOCK_M": bm}, torch.rand(T, generator=g, device=gpu)
+    for weights in (None, tw):
+        for packed in (False, True):
+            out = torch.zeros(T, N, dtype=BF16, device=gpu)
+            if packed:
+                KG.moe_gemm_packed(a, 1, KG.pack_w512(w, N, 0, False), out, weights, *lay, T, N,
+                                   False, cfg)
+            else:
+                KG.moe_gemm(a, 1, w, out, weights, *lay, T, N, 0, False, cfg)
+            assert torch.equal(out.isnan(), nan)
+    act = torch.zeros(T, N // 2, dtype=BF16, device=gpu)
+    KG.moe_gemm(a, 1, w, act, None, *lay, T, N // 2, N // 2, True, cfg)
+    assert torch.equal(act.isnan(), nan[:, :N // 2] | nan[:, N // 2:])
+
+
+@pytest.mark.parametrize("M", [40, 100, 1300])
+def test_oproj_nan_outputs(gpu, M):
+    """The same for o_proj without and with the residual (64-, 128- and 256-row tiles)."""
+    K, N = 256, 6144
+    g = torch.Generator(device=gpu).manual_seed(M)
+    a = torch.empty(M, K, dtype=BF16, device=gpu).normal_(0, 1, generator=g)
+    b = torch.empty(K, N, dtype=BF16, device=gpu).normal_(0, 1, generator=g)
+    r = torch.empty(M, N, dtype=BF16, device=gpu).normal_(0, 1, generator=g)
+    a.view(torch.int16)[[3, M - 1], [7, 200]] = torch.tensor([-1, 0x7F81], dtype=torch.int16,
+                                                             device=gpu)
+    r.view(torch.int16)[5, 77] = -63
+    nan = torch.zeros(M, N, dtype=torch.bool, device=gpu)
+    nan[[3, M - 1]] = True
+    out = torch.zeros(M, N, dtype=BF16, device=gpu)
+    KO.gemm_launch(a, b, out, None, {}, False, False)
+    assert torch.equal(out.isnan(), nan)
+    nan[5, 77] = True
+    KO.gemm_launch(a, b, out, r, {}, True, False)
+    assert torch.equal(out.isnan(), nan)
